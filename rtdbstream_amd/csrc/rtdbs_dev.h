@@ -19,7 +19,6 @@ constexpr int kCap = 512;          // candidates staged in LDS per wave
 constexpr int kMaxK = 3;           // largest stencil reach
 constexpr int kMaxRows = 49;       // (2k+1)^(dim-1) for k <= 3, dim <= 3
 constexpr int kMaxSlotBits = 24;  // slot bits of the packed key; the cell key takes the rest (<= 52)
-constexpr int kUGCells = 8;  // query cells per wave of the cell-level merge
 constexpr int kMaxBatch = 1024;
 constexpr int kMaxPerCu = 1024;  // largest workgroups-per-CU setting of a persistent grid
 constexpr int kCandPad = 4;      // floats of margin past the end of each window coordinate array
@@ -41,7 +40,6 @@ constexpr uint8_t kFlagDense = 2;
 constexpr uint8_t kCellSafe = 1;
 constexpr uint8_t kCellDense = 2;
 constexpr int kNoCore = 0x7fffffff;  // fcore of a cell without cores
-
 // Per-stream state that the device itself advances every slide.
 struct StreamMut {
     int32_t t;       // slides completed
@@ -74,7 +72,6 @@ struct StreamDev {
     float *ax, *ay, *az;
     // stride: sorted tiles (keys, bkey0), then the sorted stride (B1)
     uint64_t *bkey0;
-    float *bx0, *by0, *bz0;
     uint64_t *bkey1;
     float *bx1, *by1, *bz1;
     // cell table
@@ -86,8 +83,7 @@ struct StreamDev {
     int32_t *fcore;   // W: first (minimum-slot) core position of each cell, kNoCore if none
     // clustering
     uint8_t *flags;   // W: kFlagCore | kFlagDense
-    int32_t *parent;  // W: union-find over positions, root = minimum slot
-    int32_t *rep;     // W: union-find element of each position (cell-parallel path)
+    uint64_t *uf;     // 2W: union-find entries of cells [0, W) and of unsafe cells' cores, W + position
     int32_t *tile_a;  // ceil(W/kWTile): survivors per tile
     int32_t *tile_b;  // ceil(W/kWTile): cell starts per tile
 };
@@ -104,11 +100,13 @@ struct BatchArgs {
     const int32_t *pre_chunk;  // n+1 prefix of ceil(W/kChunk)
     unsigned long long *stats; // n * kNumStats per-stream counters, null when off
     int32_t *cell_pre;         // n+1 prefix of cells per stream (written by k_rows)
+    int32_t *ctile_pre;        // n+1 prefix of cell tiles (cell_tile cells each) per stream (written by k_rows)
+    int32_t cell_tile;         // cells per wave item of the merge of safe cells, 1..64
     int32_t xcd_groups;        // kXcd* bits: kernels whose XCDs each take one contiguous range of work
 };
 
 // BatchArgs::xcd_groups bits
-constexpr int32_t kXcdUnion = 1;         // k_union
+constexpr int32_t kXcdUnion = 1;         // k_merge_cells and k_union
 constexpr int32_t kXcdBorderPoints = 2;  // k_border_points
 
 // Kernel launchers (rtdbs_kernels.hip). All enqueue on `st` and return the
@@ -118,13 +116,14 @@ struct LaunchShape {
     int32_t wtiles;   // total window tiles
     int32_t chunks;   // total chunks
     int32_t rows_blocks;     // 256-thread blocks for the row kernel
-    int32_t cell_blocks;     // one-wave blocks for the persistent cell kernels
     int32_t lpq;             // lanes per query of the point-parallel count (1, 2 or 4)
     int32_t lpq_border;      // lanes per query of the point-parallel output kernel
     int32_t cellpar_blocks;  // blocks of the cell-parallel count and border kernels
     int32_t cellpar;         // 1: cell-parallel output kernel, 0: point-parallel
     int32_t count_cell;      // 1: cell-parallel range count (writes fcore and rep), 0: point-parallel
-    int32_t union_cells;     // point-parallel path: 1 cell-level merge kernels, 0 the cell-parallel merge
+    int32_t link;            // 1: some stream has safe cells: merged by k_merge_cells
+    int32_t unsafe;          // 1: some stream has none (reach 1): merged by k_union
+    int32_t link_blocks;     // blocks of k_merge_cells and k_cell_cores
     int32_t rank_split;      // 1: stride rank with 64-key blocks (small strides), 0: 256-key blocks
     int32_t border_regroup;  // point-parallel outputs: 1 one lane per core, non-cores regrouped onto 4 lanes
 };

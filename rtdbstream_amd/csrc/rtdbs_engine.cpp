@@ -69,12 +69,6 @@ static uint64_t next_generation() {
     return g.fetch_add(1);
 }
 
-static uint32_t next_pow2(uint64_t v) {
-    uint64_t p = 64;
-    while (p < v) p <<= 1;
-    return (uint32_t)p;
-}
-
 static int ceil_log2(int64_t v) {
     int b = 0;
     while ((int64_t(1) << b) < v) b++;
@@ -119,8 +113,8 @@ int validate_params(const rtdbs_params *p) {
 // Buffer layout of one stream's device arena.
 struct Layout {
     size_t off_mut, off_skey, off_sx, off_sy, off_sz, off_akey, off_ax, off_ay, off_az;
-    size_t off_bkey0, off_bx0, off_by0, off_bz0, off_bkey1, off_bx1, off_by1, off_bz1;
-    size_t off_cstart, off_ckey, off_pcell, off_rows, off_cflag, off_fcore, off_flags, off_parent, off_rep,
+    size_t off_bkey0, off_bkey1, off_bx1, off_by1, off_bz1;
+    size_t off_cstart, off_ckey, off_pcell, off_rows, off_cflag, off_fcore, off_flags, off_uf,
         off_tile_a, off_tile_b, off_in, off_label, off_cid;
     size_t total;
 };
@@ -149,9 +143,6 @@ static Layout make_layout(const rtdbs_params &p, int R) {
     L.off_ay = d > 1 ? take(wc) : 0;
     L.off_az = d > 2 ? take(wc) : 0;
     L.off_bkey0 = take(S * 8);
-    L.off_bx0 = take(S * 4);
-    L.off_by0 = d > 1 ? take(S * 4) : 0;
-    L.off_bz0 = d > 2 ? take(S * 4) : 0;
     L.off_bkey1 = take(S * 8);
     L.off_bx1 = take(S * 4);
     L.off_by1 = d > 1 ? take(S * 4) : 0;
@@ -163,8 +154,7 @@ static Layout make_layout(const rtdbs_params &p, int R) {
     L.off_cflag = take(W);
     L.off_fcore = take(W * 4);
     L.off_flags = take(W);
-    L.off_parent = take(W * 4);
-    L.off_rep = take(W * 4);
+    L.off_uf = take(2 * W * 8);
     L.off_tile_a = take(ntile * 4);
     L.off_tile_b = take(ntile * 4);
     L.off_in = take(W * d * 4);
@@ -261,9 +251,6 @@ extern "C" int rtdbs_stream_create(const rtdbs_params *params, rtdbs_stream **ou
     D.ay = f(L.off_ay, d > 1);
     D.az = f(L.off_az, d > 2);
     D.bkey0 = (uint64_t *)(A + L.off_bkey0);
-    D.bx0 = f(L.off_bx0, true);
-    D.by0 = f(L.off_by0, d > 1);
-    D.bz0 = f(L.off_bz0, d > 2);
     D.bkey1 = (uint64_t *)(A + L.off_bkey1);
     D.bx1 = f(L.off_bx1, true);
     D.by1 = f(L.off_by1, d > 1);
@@ -275,8 +262,7 @@ extern "C" int rtdbs_stream_create(const rtdbs_params *params, rtdbs_stream **ou
     D.cflag = (uint8_t *)(A + L.off_cflag);
     D.fcore = (int32_t *)(A + L.off_fcore);
     D.flags = (uint8_t *)(A + L.off_flags);
-    D.parent = (int32_t *)(A + L.off_parent);
-    D.rep = (int32_t *)(A + L.off_rep);
+    D.uf = (uint64_t *)(A + L.off_uf);
     D.tile_a = (int32_t *)(A + L.off_tile_a);
     D.tile_b = (int32_t *)(A + L.off_tile_b);
     s->d_in = (float *)(A + L.off_in);
@@ -512,8 +498,9 @@ static int batch_alloc(rtdbs_batch *b) {
     const size_t pre_b = ((size_t)4 * (n + 1) * 4 + 255) & ~size_t(255);
     const size_t cnt_b = ((size_t)n * kNumStats * 8 + 255) & ~size_t(255);
     const size_t cpre_b = ((size_t)(n + 1) * 4 + 255) & ~size_t(255);
-    HIPCHK(hipMalloc((void **)&b->dmem, desc_b + io_b + pre_b + cnt_b + cpre_b));
+    HIPCHK(hipMalloc((void **)&b->dmem, desc_b + io_b + pre_b + cnt_b + 2 * cpre_b));
     b->d_cell_pre = (int32_t *)(b->dmem + desc_b + io_b + pre_b + cnt_b);
+    b->d_ctile_pre = (int32_t *)(b->dmem + desc_b + io_b + pre_b + cnt_b + cpre_b);
     b->d_desc = (StreamDev *)b->dmem;
     b->d_io = (IO *)(b->dmem + desc_b);
     b->d_pre = (int32_t *)(b->dmem + desc_b + io_b);
@@ -609,10 +596,6 @@ static int env_int(const char *name, int def, int lo, int hi) {
 // and border kernels.
 constexpr long long kCellParMaxPoints = 1000000;
 
-// One-wave workgroups per CU for the persistent cell-level merge
-// (RTDBS_WAVES_PER_CU overrides, 1..64).
-static int waves_per_cu() { return env_int("RTDBS_WAVES_PER_CU", 16, 1, 64); }
-
 // Uploads descriptors and prefix tables; drops a captured graph. Called when
 // the batch is built and whenever a member stream was re-initialised.
 int refresh_batch(rtdbs_batch *b) {
@@ -674,9 +657,6 @@ int refresh_batch(rtdbs_batch *b) {
     // point-parallel; otherwise as the output kernel)
     const int cmode = env_int("RTDBS_COUNT_MODE", 0, 0, 2);
     b->shape.count_cell = cmode ? (cmode == 1) : b->shape.cellpar;
-    // the cell-parallel merge also wins in large batches (RTDBS_UNION_CELLS=1
-    // selects the older cell-level merge kernels there)
-    b->shape.union_cells = env_int("RTDBS_UNION_CELLS", 0, 0, 1);
     // cell-parallel grid: 16 blocks per CU while the launch is small; 32 for
     // large batches, where it carries the merge alone (64 streams: 455 ->
     // ~400 us). RTDBS_CELLPAR_PER_CU overrides.
@@ -685,8 +665,18 @@ int refresh_batch(rtdbs_batch *b) {
     b->shape.cellpar_blocks = (int)std::max(
         1ll, std::min((long long)device_cus() * env_int("RTDBS_CELLPAR_PER_CU", cp_def, 1, kMaxPerCu),
                       (cells_total + 3) / 4));
-    b->shape.cell_blocks = (int)std::max(
-        1ll, std::min((long long)device_cus() * waves_per_cu(), (cells_total + kUGCells - 1) / kUGCells));
+    // merge: streams with safe cells by links and joins of cells, streams of
+    // reach 1, which have none, core by core
+    b->shape.link = b->shape.unsafe = 0;
+    for (int i = 0; i < n; i++) (b->streams[i]->dense_ok ? b->shape.link : b->shape.unsafe) = 1;
+    // Cells per wave of the merge: small tiles keep a latency-bound launch's
+    // waves short (100,000 3-D points: 8 cells 27 us, 64 cells 38), large ones
+    // fill the lanes where waves abound (3.2 M points of 64 streams: 64 cells 138
+    // us, 16 cells 234; 338,000 points of 16 streams: 32 cells best by 2-6%).
+    // RTDBS_CELL_TILE overrides.
+    const int ctile = env_int("RTDBS_CELL_TILE", cells_total <= 200000 ? 8 : (cells_total <= 600000 ? 32 : 64), 1, 64);
+    b->shape.link_blocks =
+        (int)std::max(1ll, std::min((long long)device_cus() * 16, (cells_total + 4 * ctile - 1) / (4 * ctile)));
     // lanes per query: enough threads to cover the device several times over,
     // unless a single stream asks for a tuned setting
     const long long lanes_wanted = (long long)device_cus() * 32 * 64 * 4;
@@ -716,6 +706,8 @@ int refresh_batch(rtdbs_batch *b) {
     a.pre_itile = b->d_pre + 3 * (n + 1);
     a.stats = b->stats_on ? b->d_stats : nullptr;
     a.cell_pre = b->d_cell_pre;
+    a.ctile_pre = b->d_ctile_pre;
+    a.cell_tile = ctile;
     // XCD-grouped work order: in large batches for the merge and the
     // point-parallel output kernel, where it pays (RTDBS_XCD_GROUPS sets the
     // kXcd* bits)

@@ -49,6 +49,7 @@ struct rtdbs_batch {
     bool stats_on = false;
     int64_t stats_slides = 0;
     int32_t *d_cell_pre = nullptr;
+    int32_t *d_ctile_pre = nullptr;
     rtdbs::IO *h_io = nullptr;  // pinned mirror of d_io
     bool io_valid = false;
     rtdbs::StreamDev *h_desc = nullptr;  // pinned mirrors of the descriptor and prefix tables

@@ -3,8 +3,8 @@
 // One slide of every stream in a batch is eight launches:
 //   sort_expire (stride sort in runs + survivors per window tile) ->
 //   rank (stride rank merge + survivor compaction) -> merge_final -> cells ->
-//   rows -> count -> union -> border (outputs)
-// (large batches: count_points -> fcore -> rep -> union -> border_points).
+//   rows -> count -> merge_cells -> border (outputs)
+// (large batches: count_points -> cell_cores -> merge_cells -> border_regroup).
 // Each kernel covers all streams of the batch in one launch: a block finds its
 // stream from prefix tables of per-stream work units (tiles of positions,
 // 64-position chunks) or, for the cell kernels whose sizes are only known on
@@ -786,9 +786,7 @@ __global__ __launch_bounds__(kTileThreads) void k_merge_final(BatchArgs a) {
 // Cell table: ordered compaction of run starts -> cstart/ckey and position ->
 // cell. Replaces compute_offsets_of_cells + thrust_sort
 // (aabb.cu:377-410, thrust_helper.cu:16-19): the order comes from the scan,
-// so no sort and no host round trip (dbscan.cpp:549) are needed. Also resets
-// the union-find (every slot its own root) in index order, coalesced, rather
-// than slot by slot from the count kernels.
+// so no sort and no host round trip (dbscan.cpp:549) are needed.
 __global__ __launch_bounds__(kTileThreads) void k_cells(BatchArgs a) {
     __shared__ int lds4[4];
     const int g = blockIdx.x;
@@ -824,7 +822,6 @@ __global__ __launch_bounds__(kTileThreads) void k_cells(BatchArgs a) {
         const int rank = block_rank_flags(f, &tot, lds4);
         if (valid) {
             S.pcell[p] = base + run + rank + (f ? 1 : 0) - 1;
-            S.parent[p] = p;  // union-find over slots [0, W), each its own root; written in order here
         }
         if (f) {
             const int c = base + run + rank;
@@ -863,7 +860,6 @@ struct RowsView {
     gptr<const int32_t> cstart;
     gptr<uint64_t> rows;  // int2 (first, end) per stencil row, as one word
     gptr<uint8_t> cflag;
-    gptr<int32_t> fcore;
     int64_t n0, n1, n2;
     int k, R, dim, min_pts, dense_ok, ncell;
 };
@@ -874,7 +870,6 @@ __device__ __forceinline__ RowsView rows_view(const StreamDev &S) {
     v.cstart = gl(ldc(S.cstart));
     v.rows = gl((uint64_t *)ldc(S.rows));
     v.cflag = gl(ldc(S.cflag));
-    v.fcore = gl(ldc(S.fcore));
     v.n0 = ldc(S.n[0]);
     v.n1 = ldc(S.n[1]);
     v.n2 = ldc(S.n[2]);
@@ -1075,7 +1070,6 @@ __device__ __forceinline__ void rows_tile(const RowsView &V, int t, int g, uint6
             V.rows[(size_t)c * V.R + r] = row;
             if (r == 0) {
                 V.cflag[c] = cell_class(V, i0, i1, i2, c);
-                V.fcore[c] = kNoCore;
             }
         }
     }
@@ -1083,30 +1077,32 @@ __device__ __forceinline__ void rows_tile(const RowsView &V, int t, int g, uint6
 }
 
 // Persistent: walks the device-side list of (stream, 64-cell tile, row group)
-// items, one per wave. Block 0 also publishes the per-stream prefix of cell
-// counts for the cell kernels.
+// items, one per wave. One block more than the walk needs publishes the
+// per-stream prefixes of cells and of cell tiles for the later kernels, over
+// all its threads.
 __global__ __launch_bounds__(kTileThreads) void k_rows(BatchArgs a) {
     __shared__ long long pre[kMaxBatch + 1];
     __shared__ long long tmp4[4];
     __shared__ uint64_t lkey[kRowWaves][kRowCap];
     __shared__ int32_t lcs[kRowWaves][kRowCap + 1];
+    const int nb = gridDim.x - 1;  // blocks of the walk
+    if ((int)blockIdx.x == nb) {
+        block_stream_prefix(a.n, pre, tmp4, [&](int i) { return (long long)a.s[i].mut->ncell; });
+        for (int i = threadIdx.x; i <= a.n; i += kTileThreads) a.cell_pre[i] = (int32_t)pre[i];
+        __syncthreads();
+        block_stream_prefix(a.n, pre, tmp4, [&](int i) {
+            return (long long)((a.s[i].mut->ncell + a.cell_tile - 1) / a.cell_tile);
+        });
+        for (int i = threadIdx.x; i <= a.n; i += kTileThreads) a.ctile_pre[i] = (int32_t)pre[i];
+        return;
+    }
     block_stream_prefix(a.n, pre, tmp4, [&](int i) {
         const StreamDev &S = a.s[i];
         return (long long)((S.mut->ncell + kRowTile - 1) / kRowTile) * rows_groups(S.dim, S.k, S.R);
     });
-    if (blockIdx.x == 0) {
-        long long run = 0;
-        if (threadIdx.x == 0) {
-            a.cell_pre[0] = 0;
-            for (int i = 0; i < a.n; i++) {
-                run += a.s[i].mut->ncell;
-                a.cell_pre[i + 1] = (int32_t)run;
-            }
-        }
-    }
     const long long total = pre[a.n];
     const int wv = uni(threadIdx.x >> 6);
-    for (long long wi = (long long)blockIdx.x * kRowWaves + wv; wi < total; wi += (long long)gridDim.x * kRowWaves) {
+    for (long long wi = (long long)blockIdx.x * kRowWaves + wv; wi < total; wi += (long long)nb * kRowWaves) {
         const int s = uni(find_stream(pre, a.n, wi));
         const RowsView V = rows_view(a.s[s]);
         const int local = uni((int)(wi - pre[s]));
@@ -1122,34 +1118,6 @@ __global__ __launch_bounds__(kTileThreads) void k_rows(BatchArgs a) {
 // the device-side cell list in a persistent loop. The candidates of a cell
 // are the concatenation of its stencil rows; lanes 0..R-1 hold one row each.
 
-// Index r of the row holding candidate j (largest r < R with pre(r) <= j).
-// Every lane takes part; j may differ per lane.
-__device__ __forceinline__ int row_of(int pre, int R, int j) {
-    int lo = 0, hi = R;
-#pragma unroll
-    for (int it = 0; it < 6; it++) {
-        const int mid = (lo + hi) >> 1;
-        const int pm = __shfl(pre, mid);
-        if (hi - lo > 1) {
-            if (pm <= j) lo = mid;
-            else hi = mid;
-        }
-    }
-    return lo;
-}
-
-struct CellCtx {
-    int s, c;
-};
-
-__device__ __forceinline__ CellCtx cell_of(const BatchArgs &a, int gc) {
-    CellCtx x;
-    x.s = find_stream_c(a.cell_pre, a.n, gc);
-    x.c = gc - ldc(a.cell_pre[x.s]);
-    return x;
-}
-
-
 struct ChunkCtx {
     int s, p0, p1;
 };
@@ -1161,15 +1129,6 @@ __device__ __forceinline__ ChunkCtx chunk_of(const BatchArgs &a, int g) {
     x.p0 = (g - ldc(a.pre_chunk[x.s])) * kChunk;
     x.p1 = min(x.p0 + kChunk, W);
     return x;
-}
-
-// The union-find element (a slot) representing a core: the slot of the first
-// core of its cell when the cell is safe (all its points are within eps of
-// each other, so all its cores belong to one cluster), else its own slot.
-__device__ __forceinline__ int rep_slot(const StreamDev &S, int j) {
-    if (!S.dense_ok) return slot_of(S, j);
-    const int cj = S.pcell[j];
-    return slot_of(S, (S.cflag[cj] & kCellSafe) ? S.fcore[cj] : j);
 }
 
 // Wave-uniform view of one stream for the cell-parallel kernels. The
@@ -1184,8 +1143,9 @@ struct CellView {
     gptr<const uint8_t> cflag;
     gptr<const int32_t> pcell;
     gptr<uint8_t> flags;
-    gptr<int32_t> fcore, parent, rep;
-    int R, dim, min_pts;
+    gptr<int32_t> fcore;
+    gptr<uint64_t> uf;
+    int W, R, dim, min_pts;
     uint32_t smask;
     float eps2;
 };
@@ -1202,8 +1162,8 @@ __device__ __forceinline__ CellView cell_view(const StreamDev &S) {
     v.pcell = gl(ldc(S.pcell));
     v.flags = gl(ldc(S.flags));
     v.fcore = gl(ldc(S.fcore));
-    v.parent = gl(ldc(S.parent));
-    v.rep = gl(ldc(S.rep));
+    v.uf = gl(ldc(S.uf));
+    v.W = ldc(S.W);
     v.R = ldc(S.R);
     v.dim = ldc(S.dim);
     v.min_pts = ldc(S.min_pts);
@@ -1214,59 +1174,7 @@ __device__ __forceinline__ CellView cell_view(const StreamDev &S) {
 
 __device__ __forceinline__ int vslot(const CellView &V, int pos) { return (int)((uint32_t)V.skey[pos] & V.smask); }
 
-// Element at byte offset `off` of a wave-uniform array: the load takes the
-// array's scalar base and a 32-bit lane offset, with no 64-bit address
-// arithmetic per lane (window positions are below 2^24, so every offset into
-// a per-position array fits).
-template <class T>
-__device__ __forceinline__ T ldo(gptr<const T> base, uint32_t off) {
-    return *(gptr<const T>)((gptr<const char>)base + off);
-}
-template <class T>
-__device__ __forceinline__ T ldo(gptr<T> base, uint32_t off) {
-    return *(gptr<const T>)((gptr<const char>)base + off);
-}
-
 constexpr int kRowGroup = 5;  // stencil rows fetched together
-constexpr int kUnroll = 4;    // candidates fetched together
-
-// Walks the stencil candidates of cell c for one query point, kRowGroup rows
-// and kUnroll candidates per memory round trip (a thread's walk is a chain of
-// dependent loads; batching shortens it). visit(j, x, y, z) returns true to
-// stop the walk.
-// With `step` > 1 the thread takes rows first, first+step, ... only (the
-// other rows go to sibling threads of the same query).
-// Candidates at positions >= limit are skipped (rows are position ranges).
-template <class Visit>
-__device__ __forceinline__ void walk_candidates(const CellView &V, int c, Visit visit, int first = 0,
-                                                int step = 1, int limit = 0x7fffffff) {
-    const int dim = V.dim, R = V.R;
-    for (int r0 = first; r0 < R; r0 += kRowGroup * step) {
-        int rx[kRowGroup], ry[kRowGroup];
-#pragma unroll
-        for (int i = 0; i < kRowGroup; i++) {
-            const uint64_t rw = (r0 + i * step < R) ? V.rows[(size_t)c * R + r0 + i * step] : 0ull;
-            rx[i] = (int)(uint32_t)rw;
-            ry[i] = min((int)(uint32_t)(rw >> 32), limit);
-        }
-#pragma unroll
-        for (int i = 0; i < kRowGroup; i++) {
-            for (int j = rx[i]; j < ry[i]; j += kUnroll) {
-                float cx[kUnroll], cy[kUnroll], cz[kUnroll];
-#pragma unroll
-                for (int u = 0; u < kUnroll; u++) {
-                    const int jj = min(j + u, ry[i] - 1);
-                    cx[u] = V.sx[jj];
-                    cy[u] = dim > 1 ? V.sy[jj] : 0.f;
-                    cz[u] = dim > 2 ? V.sz[jj] : 0.f;
-                }
-#pragma unroll
-                for (int u = 0; u < kUnroll; u++)
-                    if (j + u < ry[i] && visit(j + u, cx[u], cy[u], cz[u])) return;
-            }
-        }
-    }
-}
 
 // Query ownership of a block of a point-parallel kernel with LPQ lanes per
 // query: block g covers chunk g / LPQ; each query is served by LPQ adjacent
@@ -1447,21 +1355,24 @@ __device__ __forceinline__ void count_cell(const CellView &V, int A, const CellH
         prefetch();
         st.add(kStatDensePoints, nA);
         const int rs = uni(rsv);
-        for (int i = lane; i < nA; i += 64) {
-            V.flags[cs + i] = kFlagCore | kFlagDense;
-            V.rep[cs + i] = rs;
+        for (int i = lane; i < nA; i += 64) V.flags[cs + i] = kFlagCore | kFlagDense;
+        if (lane == 0) {
+            V.fcore[A] = cs;
+            V.uf[A] = ufe(rs, A);
         }
-        if (lane == 0) V.fcore[A] = cs;
         return;
     }
     const bool safe = cf & kCellSafe;
     const RowWalk w0 = row_walk(lane < V.R ? h.rw : 0ull, INT_MAX);
     st.add(kStatQueries, nA);
     if (uni(wave_sum(w0.len)) < minpts) {
-        // fewer candidates than min_pts: no core (rep is read for cores only)
+        // fewer candidates than min_pts: no core
         prefetch();
         for (int i = lane; i < nA; i += 64) V.flags[cs + i] = 0;
-        if (lane == 0) V.fcore[A] = kNoCore;
+        if (lane == 0) {
+            V.fcore[A] = kNoCore;
+            V.uf[A] = kUfNone;
+        }
         return;
     }
     int fc = kNoCore, fslot = 0;
@@ -1514,7 +1425,8 @@ __device__ __forceinline__ void count_cell(const CellView &V, int A, const CellH
         }
         if (lane < nq) {
             V.flags[cs + q0 + lane] = mine >= minpts ? kFlagCore : 0;
-            if (!safe) V.rep[cs + q0 + lane] = qslot;  // unsafe cell: every core its own element
+            // unsafe cell: every core its own element
+            if (!safe) V.uf[V.W + cs + q0 + lane] = ufe(qslot, V.W + cs + q0 + lane);
         }
         const uint64_t cm = __ballot(lane < nq && mine >= minpts);
         if (fc == kNoCore && cm != 0ull) {
@@ -1525,10 +1437,10 @@ __device__ __forceinline__ void count_cell(const CellView &V, int A, const CellH
     };
     block(0, true);
     for (int q0 = 64; q0 < nA; q0 += 64) block(q0, false);
-    if (lane == 0) V.fcore[A] = fc;  // first (minimum-slot) core: the cell's representative
-    // safe cell: one union-find element, the representative's slot
-    if (safe)
-        for (int i = lane; i < nA; i += 64) V.rep[cs + i] = fc != kNoCore ? fslot : 0;
+    if (lane == 0) {
+        V.fcore[A] = fc;  // first (minimum-slot) core: the cell's representative
+        V.uf[A] = fc == kNoCore ? kUfNone : (safe ? ufe(fslot, A) : kUfUnsafe);
+    }
 }
 
 // One wave per cell in a grid-stride walk over all cells of the launch; the
@@ -1557,24 +1469,23 @@ __global__ __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu
             stats_stream(a, st, s);
             count_cell(cell_view(a.s[s]), c, h, st, prefetch);
             if (gn >= total) break;
-            gc = gn;
-            s = sn;
-            c = cn;
+            // (moved to scalar registers again: the compiler does not carry that
+            // they are uniform around the loop, and would read the descriptor
+            // and search the streams with vector loads)
+            gc = uni(gn);
+            s = uni(sn);
+            c = uni(cn);
             h = hn;
         }
     }
     stats_flush(a, st);
 }
 
-// Root of x's union-find tree, read only (no path halving): for kernels that
-// run after the merge has finished, when the trees no longer change.
-__device__ __forceinline__ int uf_root(const int32_t *parent, int x) {
-    int p = uf_load(parent + x);
-    while (p != x) {
-        x = p;
-        p = uf_load(parent + x);
-    }
-    return x;
+// Cluster id of the core at position p of cell c, whose entry is e: the slot
+// of its element's root. For kernels that run after the merge.
+__device__ __forceinline__ int core_cid(const CellView &V, uint64_t e, int p) {
+    if (e == kUfUnsafe) e = V.uf[V.W + p];
+    return ufe_slot(ufe_root(V.uf, e));
 }
 
 // Outputs of one cell, after the merge (the reference's post_cluster_t,
@@ -1590,10 +1501,12 @@ __device__ void output_cell(const BatchArgs &a, int s, const CellView &V, const 
     const int lane = lane_id();
     const int dim = V.dim;
     const float e2 = V.eps2;
-    const int32_t *parent = ldc(a.s[s].parent);
     const int cfv = V.cflag[A], csv = V.cstart[A], cev = V.cstart[A + 1];
+    const uint64_t ev = V.uf[A];
     const uint64_t rw = row_word(V, A);
     arrived(rw);
+    // a safe cell's cores share one root, found once
+    const int cidA = ufe_is(ev) ? core_cid(V, ev, 0) : 0;
     if (A == 0 && lane == 0) {
         StreamMut *m = ldc(a.s[s].mut);
         if (a.stats) a.stats[(size_t)s * kNumStats + kStatCells] += (unsigned long long)m->ncell;
@@ -1609,19 +1522,17 @@ __device__ void output_cell(const BatchArgs &a, int s, const CellView &V, const 
         const int pq = cs + q0 + min(lane, nq - 1);
         const int qf = V.flags[pq];
         const uint64_t qk = V.skey[pq];
-        const int qr = V.rep[pq];
         const float qx = V.sx[pq];
         const float qy = dim > 1 ? V.sy[pq] : 0.f;
         const float qz = dim > 2 ? V.sz[pq] : 0.f;
         arrived(qk);
-        arrived(qr);
         arrived(qx);
         arrived(qy);
         arrived(qz);
         const int qslot = (int)((uint32_t)qk & V.smask);
         if (lane < nq && (qf & kFlagCore)) {
             label[qslot] = 0;
-            cidv[qslot] = uf_root(parent, qr);
+            cidv[qslot] = ev == kUfUnsafe ? core_cid(V, ev, pq) : cidA;
         }
         if (dense) continue;
         const bool isq = lane < nq && !(qf & kFlagCore);
@@ -1637,11 +1548,11 @@ __device__ void output_cell(const BatchArgs &a, int s, const CellView &V, const 
             const float cx = V.sx[pos];
             const float cy = dim > 1 ? V.sy[pos] : 0.f;
             const float cz = dim > 2 ? V.sz[pos] : 0.f;
-            const int rp = V.rep[pos];  // meaningful for cores only
+            const int pc = V.pcell[pos];
             arrived(cx);
             arrived(cy);
             arrived(cz);
-            arrived(rp);
+            arrived(pc);
             const bool core = jb + lane < end && (f & kFlagCore);
             uint64_t m = open;
             st.add(kStatBorderTests, (unsigned long long)__popcll(m) * (unsigned)min(64, end - jb));
@@ -1654,7 +1565,7 @@ __device__ void output_cell(const BatchArgs &a, int s, const CellView &V, const 
                 const bool hit = core & (sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2);
                 if (__ballot(hit) == 0ull) continue;
                 if (!have) {
-                    if (core) cid = uf_root(parent, rp);
+                    if (core) cid = core_cid(V, V.uf[pc], pos);
                     have = true;
                 }
                 const int mn = wave_min(hit ? cid : INT_MAX);
@@ -1683,33 +1594,30 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_border(BatchArgs a) {
     stats_flush(a, st);
 }
 
-// Touching (element, element) pairs of one wave, united in parallel rounds:
-// the pairs of several candidate chunks and cells - of any streams of the
-// launch - are collected in LDS and each lane then walks the union-find of
-// its pair's stream, so the dependent loads of the walks overlap instead of
-// adding up cell after cell. 320 pairs (3.75 KB per wave) still let 8 blocks
-// of 4 waves share a CU's LDS; a fuller queue flushes less often where unites
-// are many (skewed3d 429 -> 419 us, a 62-stream served batch 1084 -> 1059 us,
-// 64 streams unchanged; 384 gained more on served batches but cost 1-2% at 64
-// streams and on walks3d).
+// ---------------------------------------------------------------------------
+// Cluster merge of streams without safe cells (reach 1): every core is an
+// element.
+
+// Touching pairs of cores of one wave, united in parallel rounds: the pairs of
+// several candidate chunks and cells - of any streams of the launch - are
+// collected in LDS and each lane then walks the union-find of its pair's
+// stream, so the dependent loads of the walks overlap instead of adding up
+// cell after cell.
 constexpr int kEdgeCap = 320;
 
 // One cell's header as the merge needs it: stream, cell within the stream,
-// first core position (kNoCore: none, or no cell), flags and position range.
+// first core position (kNoCore: none, or no cell) and position range.
 struct CellHead {
-    int s, c, fc, cf, cs, ce;
+    int s, c, fc, cs, ce;
 };
 
 // Lane l's cell g = g0 + l * nw of a wave's grid-stride sequence: its stream
 // by a per-lane binary search over the batch's cell prefix (a small table
-// that stays in cache), then the header, all lanes' loads in one round. When
-// every lane's cell is in one stream (always for a single stream) the array
-// bases come from scalar loads of that stream's descriptor, otherwise from
-// per-lane loads of each lane's descriptor. A cell past `total` reads as a
-// cell without cores. Called by the whole wave.
+// that stays in cache), then the header, all lanes' loads in one round. A cell
+// past `total`, or of a stream with safe cells, reads as a cell without cores.
 __device__ __forceinline__ CellHead cell_head(const BatchArgs &a, long long g, int total) {
-    CellHead h{0, 0, kNoCore, 0, 0, 0};
-    const bool valid = g < total;
+    CellHead h{0, 0, kNoCore, 0, 0};
+    bool valid = g < total;
     const gptr<const int32_t> pre = gl((const int32_t *)a.cell_pre);
     int lo = 0, hi = a.n, plo = 0;  // pre[0] = 0
     while (valid && hi - lo > 1) {
@@ -1724,37 +1632,23 @@ __device__ __forceinline__ CellHead cell_head(const BatchArgs &a, long long g, i
     }
     h.s = lo;
     h.c = valid ? (int)(g - plo) : 0;
-    const int s0 = uni(h.s);  // lane 0's cell is valid
-    gptr<const int32_t> fcore, cstart;
-    gptr<const uint8_t> cflag;
-    if (__ballot(valid && h.s != s0) == 0ull) {
-        const StreamDev &S = a.s[s0];
-        fcore = gl((const int32_t *)ldc(S.fcore));
-        cflag = gl((const uint8_t *)ldc(S.cflag));
-        cstart = gl((const int32_t *)ldc(S.cstart));
-    } else {
-        const gptr<const StreamDev> sd = gl(a.s) + h.s;
-        fcore = gl((const int32_t *)sd->fcore);
-        cflag = gl((const uint8_t *)sd->cflag);
-        cstart = gl((const int32_t *)sd->cstart);
-    }
+    const gptr<const StreamDev> sd = gl(a.s) + h.s;
+    valid = valid && !sd->dense_ok;
     if (valid) {
-        h.fc = fcore[h.c];
-        h.cf = cflag[h.c];
-        h.cs = cstart[h.c];
-        h.ce = cstart[h.c + 1];
+        h.fc = gl((const int32_t *)sd->fcore)[h.c];
+        h.cs = gl((const int32_t *)sd->cstart)[h.c];
+        h.ce = gl((const int32_t *)sd->cstart)[h.c + 1];
     }
     return h;
 }
 
 // Lane j's header, wave-uniform.
 __device__ __forceinline__ CellHead lane_head(const CellHead &m, int j) {
-    return CellHead{lane_i(m.s, j), lane_i(m.c, j), lane_i(m.fc, j), lane_i(m.cf, j), lane_i(m.cs, j),
-                    lane_i(m.ce, j)};
+    return CellHead{lane_i(m.s, j), lane_i(m.c, j), lane_i(m.fc, j), lane_i(m.cs, j), lane_i(m.ce, j)};
 }
 
 struct Edge {
-    int x, y;  // union-find elements (slots)
+    int x, y;  // union-find elements
     int s;     // stream
 };
 
@@ -1766,71 +1660,36 @@ struct EdgeBuf {
 __device__ __forceinline__ void edge_flush(const BatchArgs &a, EdgeBuf &eb) {
     for (int i = lane_id(); i < eb.n; i += 64) {
         const Edge e = eb.e[i];
-        uf_unite(ldc(a.s[e.s].parent), e.x, e.y);
+        ufe_unite(gl(ldc(a.s[e.s].uf)), e.x, e.y);
     }
     eb.n = 0;
 }
 
-// Queues (target, rep) for every lane that wants it, once per run of lanes
-// holding the same representative (a safe cell's points are adjacent in a
-// candidate chunk and share one representative).
 template <class ST>
-__device__ __forceinline__ void unite_once_per_rep(const BatchArgs &a, EdgeBuf &eb, int s, bool want, int rep,
-                                                   int target, ST &st) {
-    const int lane = lane_id();
+__device__ __forceinline__ void edge_push(const BatchArgs &a, EdgeBuf &eb, int s, bool want, int x, int y, ST &st) {
     const uint64_t m = __ballot(want);
     if (m == 0ull) return;
-    const uint64_t below = m & ((1ull << lane) - 1ull);
-    const int prev = below ? 63 - __clzll((long long)below) : lane;
-    const int prep = __shfl(rep, prev);
-    const bool first = want && (below == 0ull || prep != rep);
-    const uint64_t fm = __ballot(first);
-    const int nf = __popcll(fm);
-    st.add(kStatMergePairs, __popcll(m));
-    st.add(kStatUnites, nf);
-    if (eb.n + nf > kEdgeCap) edge_flush(a, eb);
-    if (first) eb.e[eb.n + __popcll(fm & ((1ull << lane) - 1ull))] = Edge{target, rep, s};
-    eb.n += nf;
+    const int n = __popcll(m);
+    st.add(kStatMergePairs, n);
+    st.add(kStatUnites, n);
+    if (eb.n + n > kEdgeCap) edge_flush(a, eb);
+    if (want) eb.e[eb.n + __popcll(m & ((1ull << lane_id()) - 1ull))] = Edge{x, y, s};
+    eb.n += n;
 }
 
-// Candidate positions before which a safe cell's merge goes over candidate
-// cells first (below it, scanning the positions costs fewer round trips).
-constexpr int kCellLevelMin = 192;
-
-// Cluster merge (the reference's __raygen__cluster + unite,
-// dbscan.cu:279-321,354-394,9-43), cell-parallel: one wave per cell A with
-// cores. Its candidates are the stencil positions before A's own first
-// position - exactly the points of the stencil cells ordered before A, so each
-// unordered pair of cells is tested once, from its later cell - loaded 64 at
-// a time, coalesced. A safe cell A (all its points within eps of each other)
-// is one union-find element, its representative: a candidate core within eps
-// of any core of A joins it. The cores of an unsafe cell are separate
-// elements, and the cell's own earlier points are candidates too. A
-// candidate's element is its safe cell's representative or its own slot.
-//
-// A safe cell with many candidates (dense regions) goes over its candidate
-// cells first, 64 per round: one safe candidate cell joins A as soon as its
-// first core is within eps of a core of A - one test per cell pair instead of
-// a scan of the cell's points, which is all the merge needs (the analogue of
-// the reference's dense-cell spheres, dbscan.cu:378-393). Only the candidate
-// cells not settled that way (unsafe cells, whose cores are separate
-// elements, and safe cells whose first core is out of reach) have their
-// points scanned.
+// The cores of cell A against the stencil's cores before them in the window
+// (the reference's __raygen__cluster + unite, dbscan.cu:279-321,354-394,9-43),
+// one wave per cell: the candidates 64 at a time, coalesced, each core tested
+// against all of them with one ballot. The stencil rows (rw, lane r: row r)
+// came in with the previous cell.
 template <class ST>
 __device__ void union_cell(const BatchArgs &a, int s, const CellView &V, const CellHead &h, ST &st, EdgeBuf &eb,
                            uint64_t rw) {
     const int lane = lane_id();
     const int dim = V.dim;
     const float e2 = V.eps2;
-    // the header comes screened (cell_head) and the stencil rows (rw, lane r:
-    // row r, every lane loaded) came in with the previous cell; the first
-    // queries and the first candidate chunk load in one round, then each
-    // further chunk is a round of its own
-    const bool safeA = h.cf & kCellSafe, denseA = h.cf & kCellDense;
     const int cs = h.cs, nA = h.ce - h.cs;
-    const RowWalk w0 = row_walk(lane < V.R ? rw : 0ull, safeA ? cs : cs + nA);
-    if (w0.rest == 0ull) return;
-    const bool by_cells = safeA && uni(wave_sum(w0.len)) >= kCellLevelMin;
+    const RowWalk w0 = row_walk(lane < V.R ? rw : 0ull, cs + nA);
     for (int q0 = 0; q0 < nA; q0 += 64) {
         const int nq = min(64, nA - q0);
         const int pq = cs + q0 + min(lane, nq - 1);
@@ -1838,161 +1697,28 @@ __device__ void union_cell(const BatchArgs &a, int s, const CellView &V, const C
         const float qx = V.sx[pq];
         const float qy = dim > 1 ? V.sy[pq] : 0.f;
         const float qz = dim > 2 ? V.sz[pq] : 0.f;
-        const int qslot = V.rep[pq];  // read for the cores of unsafe cells: the point's own slot
-        // the point scan's first chunk, in the same round (not for the
-        // cell-level pass, which scans other walks)
-        RowWalk w1 = w0;
-        int end1 = 0;
-        const int pos1 = walk_chunk(w1, 0, &end1);
-        const int f1 = by_cells ? 0 : V.flags[pos1];
-        const float x1 = by_cells ? 0.f : V.sx[pos1];
-        const float y1 = by_cells || dim < 2 ? 0.f : V.sy[pos1];
-        const float z1 = by_cells || dim < 3 ? 0.f : V.sz[pos1];
-        const int r1 = by_cells ? 0 : V.rep[pos1];
-        arrived(qx);
-        arrived(qy);
-        arrived(qz);
-        arrived(qslot);
-        arrived(x1);
-        arrived(y1);
-        arrived(z1);
-        arrived(r1);
-        // a safe cell's element: its representative's slot, which every
-        // position of the cell holds in rep - lane 0's query slot, so it comes
-        // with the queries instead of a round trip of its own (unsafe cells:
-        // each core its own slot, repA unused)
-        const int repA = lane_i(qslot, 0);
-        const bool qcore = lane < nq && (denseA || (qf & kFlagCore));
-        const uint64_t qm = __ballot(qcore);
+        const uint64_t qm = __ballot(lane < nq && (qf & kFlagCore));
         if (qm == 0ull) continue;
-        // The cores qm of this block against candidate chunk [jb, jb + 64) of
-        // a walk whose candidates end at `end`.
-        auto test = [&](const int jb, const int end, const int pos, const int f, const float cx, const float cy,
-                        const float cz, const int rp) __attribute__((always_inline)) {
-                const bool bcore = jb + lane < end && (f & kFlagCore);
-                const uint64_t bm = __ballot(bcore);
-                if (bm == 0ull) return;
-                const int rep = bcore ? rp : 0;
-                const unsigned chunk = (unsigned)min(64, end - jb);
-                uint64_t m = qm;
-                if (safeA) {
-                    // lanes holding one element form a run (a safe cell's points are
-                    // adjacent); one touching lane settles its whole run
-                    const int prev_rep = prev_lane(rep);  // every lane takes part in the moves
-                    const int prev_core = prev_lane((int)bcore);
-                    const uint64_t starts = __ballot(lane == 0 || prev_rep != rep || !prev_core);
-                    const uint64_t after = starts & ~((2ull << lane) - 1ull);  // run starts above this lane
-                    const uint64_t upto = after ? (after & (~after + 1ull)) - 1ull : ~0ull;
-                    const uint64_t below = starts & ((2ull << lane) - 1ull);
-                    const uint64_t from = ~((1ull << (63 - __clzll((long long)below))) - 1ull);
-                    const uint64_t run = upto & from;  // this lane's run
-                    // touched candidates as one wave mask: the loop carries a scalar,
-                    // not a lane predicate
-                    uint64_t t = 0;
-                    while (m) {
-                        const int qi = __ffsll((unsigned long long)m) - 1;
-                        m &= m - 1;
-                        st.add(kStatMergeTests, chunk);
-                        // every lane evaluates the test, no branch per query
-                        t |= __ballot(sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2) & bm;
-                        if ((__ballot((t & run) != 0ull) | ~bm) == ~0ull) break;  // every candidate run settled
-                    }
-                    unite_once_per_rep(a, eb, s, (t >> lane) & 1ull, rep, repA, st);
-                } else {
-                    while (m) {
-                        const int qi = __ffsll((unsigned long long)m) - 1;
-                        m &= m - 1;
-                        st.add(kStatMergeTests, chunk);
-                        const bool hit = bcore & (pos < cs + q0 + qi) &
-                                         (sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2);
-                        unite_once_per_rep(a, eb, s, hit, rep, lane_i(qslot, qi), st);
-                    }
-                }
-        };
-        // the cores qm of this block against the candidate positions of walk w
-        auto scan = [&](RowWalk w) __attribute__((always_inline)) {
-            for (int jb = 0;; jb += 64) {
-                int end;
-                const int pos = walk_chunk(w, jb, &end);
-                if (jb >= end) break;
-                const int f = V.flags[pos];
-                const float cx = V.sx[pos];
-                const float cy = dim > 1 ? V.sy[pos] : 0.f;
-                const float cz = dim > 2 ? V.sz[pos] : 0.f;
-                const int rp = V.rep[pos];  // meaningful for cores only
-                arrived(cx);
-                arrived(cy);
-                arrived(cz);
-                arrived(rp);
-                test(jb, end, pos, f, cx, cy, cz, rp);
-            }
-        };
-        if (!by_cells) {
-            // the first chunk came with the queries
-            if (end1 > 0) test(0, end1, pos1, f1, x1, y1, z1, r1);
-            for (int jb = 64;; jb += 64) {
-                int end;
-                const int pos = walk_chunk(w1, jb, &end);
-                if (jb >= end) break;
-                const int f = V.flags[pos];
-                const float cx = V.sx[pos];
-                const float cy = dim > 1 ? V.sy[pos] : 0.f;
-                const float cz = dim > 2 ? V.sz[pos] : 0.f;
-                const int rp = V.rep[pos];
-                arrived(cx);
-                arrived(cy);
-                arrived(cz);
-                arrived(rp);
-                test(jb, end, pos, f, cx, cy, cz, rp);
-            }
-            continue;
-        }
-        // candidate cells: row r (lane r) covers positions [rx, rx + len), all
-        // before cs, i.e. the cells pcell[rx] .. pcell[rx + len - 1] (< A)
-        const int clo = w0.len > 0 ? V.pcell[w0.rx] : 0;
-        const int chi = w0.len > 0 ? V.pcell[w0.rx + w0.len - 1] + 1 : 0;
-        RowWalk cw;
-        cw.rx = clo;
-        cw.len = chi - clo;
-        cw.rest = __ballot(cw.len > 0);
+        RowWalk w = w0;
         for (int jb = 0;; jb += 64) {
-            int endc;
-            const int B = walk_chunk(cw, jb, &endc);
-            if (jb >= endc) break;
-            const bool valid = jb + lane < endc;
-            const int fb = V.fcore[B];
-            const int cfb = V.cflag[B];
-            const int bs = V.cstart[B];
-            const int be = V.cstart[B + 1];
-            arrived(fb);
-            arrived(be);
-            const bool has = valid && fb != kNoCore;
-            const int fp = has ? fb : cs;  // a valid position either way
-            const float bx = V.sx[fp];
-            const float by = dim > 1 ? V.sy[fp] : 0.f;
-            const float bz = dim > 2 ? V.sz[fp] : 0.f;
-            const int bk = V.rep[fp];  // a safe cell's element: its first core's slot
-            arrived(bx);
-            arrived(by);
-            arrived(bz);
-            arrived(bk);
-            // safe candidate cells: A's cores against each cell's first core
-            const uint64_t cand = __ballot(has && (cfb & kCellSafe));
-            uint64_t hit = 0;
-            for (uint64_t m = qm; m && hit != cand;) {
+            int end;
+            const int pos = walk_chunk(w, jb, &end);
+            if (jb >= end) break;
+            const int f = V.flags[pos];
+            const float cx = V.sx[pos];
+            const float cy = dim > 1 ? V.sy[pos] : 0.f;
+            const float cz = dim > 2 ? V.sz[pos] : 0.f;
+            arrived(cx);
+            arrived(cy);
+            arrived(cz);
+            const bool bcore = jb + lane < end && (f & kFlagCore);
+            for (uint64_t m = qm; m; m &= m - 1ull) {
                 const int qi = __ffsll((unsigned long long)m) - 1;
-                m &= m - 1;
-                st.add(kStatMergeTests, (unsigned)__popcll(cand & ~hit));
-                hit |= __ballot(sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), bx, by, bz) < e2) & cand;
+                st.add(kStatMergeTests, (unsigned)min(64, end - jb));
+                const bool hit = bcore & (pos < cs + q0 + qi) &
+                                 (sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2);
+                edge_push(a, eb, s, hit, V.W + pos, V.W + cs + q0 + qi, st);
             }
-            // a safe cell's element is its first core's slot; one lane per cell
-            unite_once_per_rep(a, eb, s, (hit >> lane) & 1ull, bk, repA, st);
-            // the cells with cores not settled: scan their points
-            RowWalk pw;
-            pw.rx = bs;
-            pw.len = (has && !((hit >> lane) & 1ull)) ? be - bs : 0;
-            pw.rest = __ballot(pw.len > 0);
-            if (pw.rest) scan(pw);
         }
     }
 }
@@ -2033,6 +1759,576 @@ __global__ __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu
     }
     edge_flush(a, eb);
     stats_flush(a, st);
+}
+
+// ---------------------------------------------------------------------------
+// Cluster merge of streams whose interior cells are safe (k*k > dim), one
+// launch over tiles of consecutive cells, a tile per wave.
+//
+// A safe cell is one union-find element, and what the merge needs is which
+// cells touch, transitively. Nearly all of that is found by very few tests:
+//   links  join every cell with at most one earlier cell on each axis, a cell
+//          whose first core is within eps of this cell's first core;
+//   joins  go over all earlier stencil cells and compare roots. Only pairs
+//          whose roots still differ are tested, in a lane where that takes few
+//          tests and otherwise by several lanes together.
+// Once every cell is linked (1.0-1.8 unites a cell), 0.03-4% of the cell pairs
+// of the 64-stream batch, of a 1 M-point window of uneven density and of
+// 100,000 trajectory points still have different roots; the one-wave-per-cell
+// kernel that this replaced tested the cores of every pair. Its times and
+// these, in us (events): 64 streams 360 and 138 (with the pass over the cells
+// that follows the point-parallel count), 1 M points 446 and 92, 100,000 1-D
+// points in dense cells 128 and 15, 100,000 trajectory points 31 and 27,
+// 10,000 2-D points 28.6 and 15; 1,000 2-D points 9 and 14, 61,503 points with
+// a third of eps per cell 24 and 27.
+//
+// What bounds it is each wave's chain of dependent loads (entry, row, the
+// row's cells, their entries and first cores, the walks to the roots, the
+// hook), so every step of it serves as many cells or pairs as it can: a
+// tile's cells without cores take no lanes, unites and pairs are queued in
+// LDS and taken 64 at a time.
+
+// The lanes of a tile's cells for which `in` holds, in order: lane i of the
+// result holds the lane of the i-th such cell (the others follow).
+__device__ __forceinline__ int tile_order(bool in, uint64_t m) {
+    const int lane = lane_id();
+    const int below = __popcll(m & ((1ull << lane) - 1ull));
+    return __builtin_amdgcn_ds_permute((in ? below : __popcll(m) + lane - below) << 2, lane);
+}
+
+__device__ __forceinline__ int from_lane(int v, int l) { return __builtin_amdgcn_ds_bpermute(l << 2, v); }
+
+__device__ __forceinline__ uint64_t from_lane64(uint64_t v, int l) {
+    const uint32_t lo = (uint32_t)from_lane((int)(uint32_t)v, l), hi = (uint32_t)from_lane((int)(uint32_t)(v >> 32), l);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// LDS written by lanes of this wave is read by others next.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// First and last cell before cell A of stencil row r (Bf > Bl: none).
+__device__ __forceinline__ void row_cells(const CellView &V, int A, uint64_t rw, int *Bf, int *Bl) {
+    const int rx = (int)(uint32_t)rw, ry = (int)(uint32_t)(rw >> 32);
+    const int f = at(V.pcell, rx), l = at(V.pcell, max(ry - 1, 0));  // an empty row is (0, 0)
+    *Bf = f;
+    *Bl = ry > rx ? min(l, A - 1) : f - 1;
+}
+
+// Pairs of elements of one stream, united 64 at a time, one per lane: the
+// walks and hooks of a tile's unites overlap instead of adding up.
+constexpr int kLinkCap = 64 * 4;  // a tile's most: 64 cells, up to 4 unites each
+
+struct LinkBuf {
+    int2 *e;  // this wave's LDS slice
+    int n;    // pairs held (uniform)
+};
+
+__device__ __forceinline__ void link_push(LinkBuf &lb, bool want, int x, int y) {
+    const uint64_t m = __ballot(want);
+    if (want) lb.e[lb.n + __popcll(m & ((1ull << lane_id()) - 1ull))] = make_int2(x, y);
+    lb.n += __popcll(m);
+}
+
+// Links of a tile's cells, lane i on the tile's i-th cell with cores. A cell
+// joins the cell with cores before it in the table when their first cores are
+// within eps (in a column that is its nearest neighbour; across columns the
+// test fails). The resulting runs need no unites: each member hooks under the
+// run's minimum slot, one atomic on its own entry. On each other axis a cell
+// joins the first cell of the stencil row one step back (nearest first) whose
+// first core is within eps, unless the cell before it in its run already did:
+// the two rows' cells are most likely one run as well.
+template <int D, class ST>
+__device__ __forceinline__ void link_tile(const CellView &V, int k, int c0, int T, int ncell, LinkBuf &lb, ST &st) {
+    const int lane = lane_id();
+    const bool valid = lane < T && c0 + lane < ncell;
+    const uint64_t w = valid ? at(V.uf, c0 + lane) : kUfNone;
+    const int fc = valid ? at(V.fcore, c0 + lane) : 0;
+    const uint64_t m = __ballot(ufe_is(w));
+    if (m == 0ull) return;
+    const int nm = __popcll(m);
+    const int order = tile_order(ufe_is(w), m);
+    const bool have = lane < nm;
+    const int A = c0 + order;
+    const uint64_t wa = from_lane64(w, order);  // (other waves may have hooked the entry already)
+    const int fa = from_lane(fc, order);  // (every lane takes part in the moves)
+    const int pa = have ? fa : 0;
+    const float ax = at(V.sx, pa);
+    const float ay = D > 1 ? at(V.sy, pa) : 0.f;
+    const float az = D > 2 ? at(V.sz, pa) : 0.f;
+    uint64_t rw[D];
+#pragma unroll
+    for (int i = 1; i < D; i++) rw[i] = have ? V.rows[(size_t)A * V.R + (i == 1 ? 1 : 2 * k + 1)] : 0ull;
+    // the cell before: lane - 1; for lane 0 the cell before the tile
+    bool b1 = false;
+    float x1 = 0.f, y1 = 0.f, z1 = 0.f;
+    if (lane == 0 && c0 > 0) {
+        b1 = ufe_is(at(V.uf, c0 - 1));
+        const int p1 = b1 ? at(V.fcore, c0 - 1) : 0;
+        x1 = at(V.sx, p1);
+        y1 = D > 1 ? at(V.sy, p1) : 0.f;
+        z1 = D > 2 ? at(V.sz, p1) : 0.f;
+    }
+    const float px = __int_as_float(prev_lane(__float_as_int(ax)));
+    const float py = __int_as_float(prev_lane(__float_as_int(ay)));
+    const float pz = __int_as_float(prev_lane(__float_as_int(az)));
+    const bool joins = have & (lane > 0) & (sqd(D, ax, ay, az, px, py, pz) < V.eps2);
+    const uint64_t lm = __ballot(joins);  // lanes that continue the run of the lane before
+    const uint64_t heads = ~lm, upto = (2ull << lane) - 1ull;
+    const int first = 63 - __clzll((long long)(heads & upto));  // (lane 0 is a head)
+    const uint64_t later = heads & ~upto;
+    const int last = later ? __ffsll((unsigned long long)later) - 2 : 63;
+    uint64_t rm = wa;  // minimum entry of the run
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t y = from_lane64(rm, max(lane - o, 0));
+        if (lane - o >= first) rm = min(rm, y);
+    }
+    rm = from_lane64(rm, last);
+    uint64_t old = rm;
+    if (have && wa != rm) old = ufe_min(V.uf + A, rm);
+    int to[D];
+    int tests = have && lane > 0;
+#pragma unroll
+    for (int i = 1; i < D; i++) {
+        int Bf, Bl;
+        row_cells(V, A, rw[i], &Bf, &Bl);
+        const int n = have ? Bl - Bf + 1 : 0;
+        const int mid = (Bf + Bl) >> 1;
+        to[i] = -1;
+        for (int u0 = 0; u0 < n && to[i] < 0; u0 += 3) {
+            bool wb[3];
+            int cb[3];
+            float bx[3], by[3], bz[3];
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const int u = min(u0 + q, n - 1);
+                const int B = cb[q] = mid + ((u & 1) ? (u + 1) >> 1 : -(u >> 1));
+                wb[q] = ufe_is(at(V.uf, B));
+                const int p = at(V.fcore, B);
+                const int pp = wb[q] ? p : 0;
+                bx[q] = at(V.sx, pp);
+                by[q] = D > 1 ? at(V.sy, pp) : 0.f;
+                bz[q] = D > 2 ? at(V.sz, pp) : 0.f;
+            }
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const bool t = (u0 + q < n) & (to[i] < 0) & wb[q];
+                tests += t;
+                if (t & (sqd(D, ax, ay, az, bx[q], by[q], bz[q]) < V.eps2)) to[i] = cb[q];
+            }
+        }
+    }
+    // (an entry that was no root any more: its ancestor joins the run)
+    link_push(lb, old != rm && ufe_idx(old) != A, ufe_idx(rm), ufe_idx(old));
+    const bool t1 = b1 & (sqd(D, ax, ay, az, x1, y1, z1) < V.eps2);
+    link_push(lb, t1, ufe_idx(rm), c0 - 1);
+    int nu = __popcll(lm) + (__ballot(t1) != 0ull);
+#pragma unroll
+    for (int i = 1; i < D; i++) {
+        const uint64_t hit = __ballot(to[i] >= 0);
+        const bool want = to[i] >= 0 && !((((hit << 1) & lm) >> lane) & 1ull);
+        link_push(lb, want, ufe_idx(rm), to[i]);
+        nu += __popcll(__ballot(want));
+    }
+    wave_sync();
+    for (int i = lane; i < lb.n; i += 64) ufe_unite(V.uf, lb.e[i].x, lb.e[i].y);
+    lb.n = 0;
+    st.add(kStatMergeTests, wave_sum(tests));
+    st.add(kStatMergePairs, nu);
+    st.add(kStatUnites, nu);
+}
+
+// Cell pairs the wave tests core by core: lane of the tile's cell A in the
+// upper 8 bits, cell B below.
+constexpr int kPairCap = 512;  // 64 rows of at most kRowCells cells, and fewer than 64 pairs left over
+constexpr int kFew = 4;  // points of a cell tested in a lane
+constexpr int kRowCells = 2 * kMaxK + 1;  // most cells of a stencil row
+
+struct PairBuf {
+    uint32_t *e;  // this wave's LDS slice
+    int n;        // pairs held (uniform)
+};
+
+__device__ __forceinline__ void pair_push(PairBuf &pb, bool want, int la, int B) {
+    const uint64_t m = __ballot(want);
+    if (want) pb.e[pb.n + __popcll(m & ((1ull << lane_id()) - 1ull))] = ((uint32_t)la << 24) | (uint32_t)B;
+    pb.n += __popcll(m);
+}
+
+// (What follows is one instance for every dimension and reach, each loop with
+// one call site: inlined per dimension it was 130 KB of code, twice the
+// instruction cache of a pair of CUs, and no faster.)
+
+// Minimum over groups of lp lanes: 8, 16 or 64 (uniform).
+__device__ __forceinline__ float group_fmin(float v, int lp) {
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) v = fminf(v, __int_as_float(xor_lane(__float_as_int(v), o)));
+    if (lp > 8) v = fminf(v, __int_as_float(xor_lane(__float_as_int(v), 8)));
+    if (lp > 16) {
+        v = fminf(v, __int_as_float(xor_lane(__float_as_int(v), 16)));
+        v = fminf(v, __int_as_float(xor_lane(__float_as_int(v), 32)));
+    }
+    return v;
+}
+
+// Gap between x and the interval [lo, -nhi].
+__device__ __forceinline__ float gap(float x, float lo, float nhi) {
+    return x < lo ? __fsub_rn(lo, x) : (x > -nhi ? __fsub_rn(x, -nhi) : 0.f);
+}
+
+// Up to kHeld points per lane of a group of lanes, with their core flags and
+// the box of the cores (upper bounds negated: one kind of reduction).
+constexpr int kHeld = 4;
+
+struct HeldCores {
+    float x[kHeld], y[kHeld], z[kHeld];
+    bool core[kHeld];
+    float lx, ly, lz, nx, ny, nz;
+};
+
+// The points at positions [c0, c1), at most lp * kHeld of them, on lp lanes.
+__device__ __forceinline__ void hold_cores(const CellView &V, int lp, bool on, int c0, int c1, HeldCores &h) {
+    const int sub = lane_id() & (lp - 1);
+    const float inf = __int_as_float(0x7f800000);
+    h.lx = h.ly = h.lz = h.nx = h.ny = h.nz = inf;
+#pragma unroll
+    for (int q = 0; q < kHeld; q++) {
+        const int i = c0 + q * lp + sub;
+        const int p = on ? min(i, c1 - 1) : 0;
+        h.x[q] = at(V.sx, p);
+        h.y[q] = V.dim > 1 ? at(V.sy, p) : 0.f;
+        h.z[q] = V.dim > 2 ? at(V.sz, p) : 0.f;
+        h.core[q] = on && i < c1 && (at(V.flags, p) & kFlagCore);
+    }
+#pragma unroll
+    for (int q = 0; q < kHeld; q++) {
+        h.lx = fminf(h.lx, h.core[q] ? h.x[q] : inf);
+        h.ly = fminf(h.ly, h.core[q] ? h.y[q] : inf);
+        h.lz = fminf(h.lz, h.core[q] ? h.z[q] : inf);
+        h.nx = fminf(h.nx, h.core[q] ? -h.x[q] : inf);
+        h.ny = fminf(h.ny, h.core[q] ? -h.y[q] : inf);
+        h.nz = fminf(h.nz, h.core[q] ? -h.z[q] : inf);
+    }
+}
+
+// Do cores of A (positions [csA, ceA)) and B touch? lp lanes a pair, at most
+// lp * kHeld points a side, all loaded in one round. Nearly all pairs that get
+// here do not touch, so A's cores are held against the box of B's cores first
+// and only those within eps of it tested against B's cores. (The rounded gap
+// between a point and the box is at most its rounded difference to any point
+// of the box, per axis, so nothing that touches is left out.) Called by the
+// whole wave; `on` marks the groups that have a pair; A is best the smaller
+// cell.
+__device__ __forceinline__ bool cells_touch(const CellView &V, int lp, bool on, int csA, int ceA, int csB, int ceB,
+                                            int &tests) {
+    const int lane = lane_id();
+    const uint64_t gm = lp == 64 ? ~0ull : ((1ull << lp) - 1ull) << (lane & ~(lp - 1));
+    HeldCores a, b;
+    hold_cores(V, lp, on, csA, ceA, a);
+    hold_cores(V, lp, on, csB, ceB, b);
+    b.lx = group_fmin(b.lx, lp);
+    b.ly = group_fmin(b.ly, lp);
+    b.lz = group_fmin(b.lz, lp);
+    b.nx = group_fmin(b.nx, lp);
+    b.ny = group_fmin(b.ny, lp);
+    b.nz = group_fmin(b.nz, lp);
+    const bool more = __ballot(on && ceB - csB > lp) != 0ull;  // a group holds more than a point of B per lane
+    // bit q: this lane's q-th point of A is a core near the box
+    uint32_t near = 0;
+#pragma unroll
+    for (int q = 0; q < kHeld; q++)
+        near |= (a.core[q] & (sqd(3, gap(a.x[q], b.lx, b.nx), gap(a.y[q], b.ly, b.ny), gap(a.z[q], b.lz, b.nz),
+                                  0.f, 0.f, 0.f) < V.eps2))
+                    ? 1u << q
+                    : 0u;
+    bool touch = false;
+    while (true) {
+        const uint64_t m = __ballot(near != 0u) & gm;  // lanes of the group with such cores
+        if (__ballot(m != 0ull) == 0ull) return touch;
+        const int l = m ? __ffsll((unsigned long long)m) - 1 : lane;
+        // this lane's next one, then the one of the group's lane l
+        const int q = __ffs(near) - 1;
+        float x = a.x[0], y = a.y[0], z = a.z[0];
+#pragma unroll
+        for (int r = 1; r < kHeld; r++) {
+            x = q == r ? a.x[r] : x;
+            y = q == r ? a.y[r] : y;
+            z = q == r ? a.z[r] : z;
+        }
+        x = __int_as_float(from_lane(__float_as_int(x), l));
+        y = __int_as_float(from_lane(__float_as_int(y), l));
+        z = __int_as_float(from_lane(__float_as_int(z), l));
+        if (lane == l) near &= near - 1u;
+        bool hit = b.core[0] & (sqd(3, x, y, z, b.x[0], b.y[0], b.z[0]) < V.eps2);
+        if (more) {
+#pragma unroll
+            for (int r = 1; r < kHeld; r++) hit |= b.core[r] & (sqd(3, x, y, z, b.x[r], b.y[r], b.z[r]) < V.eps2);
+        }
+        hit &= m != 0ull;
+        tests += m != 0ull;
+        if (__ballot(hit) & gm) {
+            touch = true;
+            near = 0;
+        }
+    }
+}
+
+// Cores of cell A against cores of cell B <= A where a cell is not safe, the
+// whole wave: every touching pair of cores unites (in A = B each pair once).
+__device__ __forceinline__ void join_cores(const CellView &V, int A, int B, bool safeA, bool safeB, int csA, int ceA,
+                                           int csB, int ceB, int &tests, int &unites) {
+    for (int pb = csB + lane_id(); pb < ceB; pb += 64) {
+        const float bx = at(V.sx, pb);
+        const float by = V.dim > 1 ? at(V.sy, pb) : 0.f;
+        const float bz = V.dim > 2 ? at(V.sz, pb) : 0.f;
+        if (!(at(V.flags, pb) & kFlagCore)) continue;
+        for (int pa = csA; pa < (A != B ? ceA : pb); pa++) {
+            tests++;
+            if ((at(V.flags, pa) & kFlagCore) && sqd(3, at(V.sx, pa), V.dim > 1 ? at(V.sy, pa) : 0.f,
+                                                 V.dim > 2 ? at(V.sz, pa) : 0.f, bx, by, bz) < V.eps2) {
+                unites++;
+                ufe_unite(V.uf, safeA ? A : V.W + pa, safeB ? B : V.W + pb);
+            }
+        }
+    }
+}
+
+// The queued pairs: 64 at a time their entries, ranges and roots, one pair
+// per lane; then those of safe cells with different roots, by the larger
+// cell's points, on 8, 16 or 64 lanes each (most cells that get here hold a
+// handful of points, and a pair's time is its chain of loads; the largest go
+// 256 by 256 points); then the pairs with an unsafe cell.
+template <class ST>
+__device__ __forceinline__ void join_flush(const CellView &V, int c0, PairBuf &pb, ST &st) {
+    const int lane = lane_id();
+    int tests = 0, unites = 0;
+    for (int i0 = 0; i0 < pb.n; i0 += 64) {
+        const uint32_t e = pb.e[min(i0 + lane, pb.n - 1)];
+        int A = c0 + (int)(e >> 24), B = (int)(e & 0xffffffu);
+        const uint64_t ea = ufe_now(V.uf, A), eb = ufe_now(V.uf, B);
+        int csA = at(V.cstart, A), ceA = at(V.cstart, A + 1), csB = at(V.cstart, B), ceB = at(V.cstart, B + 1);
+        const bool on = i0 + lane < pb.n, safe = ufe_is(ea) && ufe_is(eb);
+        bool open = on && safe;
+        if (open) open = ufe_root_now(V.uf, ea) != ufe_root_now(V.uf, eb);
+        if (open && ceA - csA > ceB - csB) {  // the smaller cell first
+            int t = A;
+            A = B;
+            B = t;
+            t = csA;
+            csA = csB;
+            csB = t;
+            t = ceA;
+            ceA = ceB;
+            ceB = t;
+        }
+        // the small pairs eight a step, the larger ones four, the rest one by one
+        const bool open8 = open && ceB - csB <= 8 * kHeld;
+        const bool open16 = open && !open8 && ceB - csB <= 16 * kHeld;
+        const uint64_t m8 = __ballot(open8), m16 = __ballot(open16);
+        uint64_t bm = __ballot(open && !open8 && !open16);
+        const int order8 = tile_order(open8, m8), order16 = tile_order(open16, m16);
+        const int n8 = __popcll(m8), n16 = __popcll(m16);
+        int a0 = 0, b0 = 0;  // the big pair's next points
+        for (int k8 = 0, k16 = 0; k8 < n8 || k16 < n16 || bm != 0ull;) {
+            const int lp = k8 < n8 ? 8 : (k16 < n16 ? 16 : 64);
+            const int g = lane / lp + (lp == 8 ? k8 : k16), n = lp == 8 ? n8 : n16;
+            const int l8 = from_lane(order8, min(g, 63)), l16 = from_lane(order16, min(g, 63));
+            const int lb = bm ? __ffsll((unsigned long long)bm) - 1 : 0;
+            const int l = lp == 8 ? l8 : (lp == 16 ? l16 : lb);
+            const bool has = lp == 64 || g < n;
+            const int x = from_lane(A, l), y = from_lane(B, l);
+            int a1 = from_lane(csA, l), a2 = from_lane(ceA, l), b1 = from_lane(csB, l), b2 = from_lane(ceB, l);
+            bool last = true;  // of this pair's steps
+            if (lp == 64) {
+                const int na = uni(a2) - uni(a1), nb = uni(b2) - uni(b1);
+                a1 += a0;
+                b1 += b0;
+                a2 = min(a1 + 64 * kHeld, a2);
+                b2 = min(b1 + 64 * kHeld, b2);
+                b0 += 64 * kHeld;
+                if (b0 >= nb) {
+                    b0 = 0;
+                    a0 += 64 * kHeld;
+                }
+                last = a0 >= na;
+            }
+            const bool touch = cells_touch(V, lp, has, a1, a2, b1, b2, tests);
+            if (touch && (lane & (lp - 1)) == 0) {
+                unites++;
+                ufe_unite(V.uf, x, y);
+            }
+            if (lp == 8) {
+                k8 += 8;
+            } else if (lp == 16) {
+                k16 += 4;
+            } else if (last || uni(touch)) {
+                bm &= bm - 1ull;
+                a0 = b0 = 0;
+            }
+        }
+        for (uint64_t m = __ballot(on && !safe); m; m &= m - 1ull) {
+            const int l = __ffsll((unsigned long long)m) - 1;
+            join_cores(V, lane_i(A, l), lane_i(B, l), lane_i(ufe_is(ea), l), lane_i(ufe_is(eb), l), lane_i(csA, l),
+                       lane_i(ceA, l), lane_i(csB, l), lane_i(ceB, l), tests, unites);
+        }
+    }
+    pb.n = 0;
+    unites = wave_sum(unites);
+    st.add(kStatMergeTests, wave_sum(tests));
+    st.add(kStatMergePairs, unites);
+    st.add(kStatUnites, unites);
+}
+
+// Joins of a tile's cells. The (cell, earlier stencil row) pairs are spread
+// over the lanes and a row's cells queued as (cell, cell) pairs; the pairs'
+// roots are then compared 64 at a time, one pair per lane (rows are mostly
+// empty and cells few, so a lane for every cell a row could hold would idle
+// 15 lanes of 16). Pairs with one root are done. The others are tested in
+// their lane: cells of up to kFew points in full, larger ones by their first
+// cores; larger cells that this does not join, and every pair with an unsafe
+// cell, go to `far`.
+template <class ST>
+__device__ __forceinline__ void join_tile(const CellView &V, int k, int c0, int T, int ncell, PairBuf &pb, PairBuf &far,
+                                          ST &st) {
+    const int lane = lane_id(), dim = V.dim;
+    const int width = 2 * k + 1;
+    const int nrow = dim == 3 ? 1 + k + k * width : (dim == 2 ? 1 + k : 1);  // rows with earlier cells
+    // x / nrow and x / width for the small x below, by multiplication
+    const int irow = 65536 / nrow + 1, iwidth = 65536 / width + 1;
+    const bool valid = lane < T && c0 + lane < ncell;
+    const uint64_t w = valid ? ufe_now(V.uf, c0 + lane) : kUfNone;
+    const uint64_t m = __ballot(w != kUfNone);
+    if (m == 0ull) return;
+    const int items = __popcll(m) * nrow;
+    const int order = tile_order(w != kUfNone, m);
+    // this lane's cell's root, compressed onto its entry; -1: an unsafe cell
+    int ra = -1;
+    if (ufe_is(w)) {
+        const uint64_t r = ufe_root_now(V.uf, w);
+        ra = ufe_idx(r);
+        if (r != w) ufe_min(V.uf + c0 + lane, r);
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (int t0 = 0; t0 < items || pb.n > 0;) {
+        if (t0 < items && pb.n < 64) {
+            const int t = min(t0 + lane, items - 1);
+            const int i = (t * irow) >> 16, e = t - i * nrow;
+            const int la = from_lane(order, i), A = c0 + la;
+            const int rA = from_lane(ra, la);
+            int r = e <= k ? max(2 * e - 1, 0) : 0;  // own plane: offset -e is stored at 2e - 1
+            if (dim == 3 && e > k) {
+                const int f = e - 1 - k, d = (f * iwidth) >> 16;  // plane -(d + 1) is group 2d + 1
+                r = (2 * d + 1) * width + f - d * width;
+            }
+            int Bf, Bl;
+            row_cells(V, A, V.rows[(size_t)A * V.R + r], &Bf, &Bl);
+            // an unsafe cell is also paired with itself, by its own column's lane
+            if (e == 0 && rA < 0) Bl = A;
+            const int n = t0 + lane < items ? Bl - Bf + 1 : 0;  // at most kRowCells
+            const uint64_t n1 = __ballot(n & 1), n2 = __ballot(n & 2), n4 = __ballot(n & 4);
+            const int at = pb.n + __popcll(n1 & below) + 2 * __popcll(n2 & below) + 4 * __popcll(n4 & below);
+            for (int u = 0; u < n; u++) pb.e[at + u] = ((uint32_t)la << 24) | (uint32_t)(Bf + u);
+            pb.n += __popcll(n1) + 2 * __popcll(n2) + 4 * __popcll(n4);
+            t0 += 64;
+            wave_sync();
+        }
+        if (pb.n >= 64 || (t0 >= items && pb.n > 0)) {
+            const int i = pb.n - 1 - lane;  // from the end: what stays needs no move
+            const uint32_t e = pb.e[max(i, 0)];
+            pb.n = max(pb.n - 64, 0);
+            const int la = (int)(e >> 24), B = (int)(e & 0xffffffu);
+            const int r0 = from_lane(ra, la);
+            const uint64_t eb = ufe_now(V.uf, B);
+            bool open = i >= 0 && eb != kUfNone && (ufe_idx(eb) != r0 || r0 < 0);
+            bool hit = false, test = false;
+            if (open && r0 >= 0 && ufe_is(eb)) {
+                const uint64_t rb = ufe_root_now(V.uf, eb), r1 = ufe_root_now(V.uf, ufe_now(V.uf, r0));
+                open = rb != r1;
+                if (open) {
+                    // all points of two cells of up to kFew, else the first cores
+                    const int A = c0 + la;
+                    const int csA = at(V.cstart, A), nA = at(V.cstart, A + 1) - csA, fA = at(V.fcore, A);
+                    const int csB = at(V.cstart, B), nB = at(V.cstart, B + 1) - csB, fB = at(V.fcore, B);
+                    const bool few = max(nA, nB) <= kFew;
+                    float ax[kFew], ay[kFew], az[kFew];
+                    bool ac[kFew];
+#pragma unroll
+                    for (int q = 0; q < kFew; q++) {
+                        const int p = few ? csA + min(q, nA - 1) : fA;
+                        ax[q] = at(V.sx, p);
+                        ay[q] = dim > 1 ? at(V.sy, p) : 0.f;
+                        az[q] = dim > 2 ? at(V.sz, p) : 0.f;
+                        ac[q] = at(V.flags, p) & kFlagCore;
+                    }
+#pragma unroll
+                    for (int q = 0; q < kFew; q++) {
+                        const int p = few ? csB + min(q, nB - 1) : fB;
+                        const float x = at(V.sx, p);
+                        const float y = dim > 1 ? at(V.sy, p) : 0.f;
+                        const float z = dim > 2 ? at(V.sz, p) : 0.f;
+                        const bool bc = at(V.flags, p) & kFlagCore;
+#pragma unroll
+                        for (int o = 0; o < kFew; o++)
+                            hit |= bc & ac[o] & (sqd(3, ax[o], ay[o], az[o], x, y, z) < V.eps2);
+                    }
+                    test = true;
+                    if (hit) ufe_unite(V.uf, ufe_idx(r1), ufe_idx(rb));
+                    open = !hit && !few;
+                }
+            }
+            const int nu = __popcll(__ballot(hit));
+            st.add(kStatMergeTests, __popcll(__ballot(test)));
+            st.add(kStatMergePairs, nu);
+            st.add(kStatUnites, nu);
+            pair_push(far, open, la, B);
+        }
+        if (far.n > kPairCap - 64 || (t0 >= items && pb.n == 0 && far.n > 0)) {
+            wave_sync();
+            join_flush(V, c0, far, st);
+        }
+    }
+}
+
+// Walks the cell tiles of the launch's streams with safe cells, one per wave:
+// tile(s, V, c0, ncell).
+template <class ST, class F>
+__device__ __forceinline__ void each_cell_tile(const BatchArgs &a, ST &st, F &&tile) {
+    const int total = uni(ldc(a.ctile_pre[a.n]));
+    const int nw = gridDim.x * kCellWaves;
+    int s = 0;
+    for (int g = uni(xcd_block(blockIdx.x, gridDim.x, a.xcd_groups & kXcdUnion) * kCellWaves + (threadIdx.x >> 6));
+         g < total; g += nw) {
+        s = uni(find_stream_from(a.ctile_pre, a.n, g, s));
+        const StreamDev &S = a.s[s];
+        if (!ldc(S.dense_ok)) continue;
+        stats_stream(a, st, s);
+        tile(S, cell_view(S), (g - uni(ldc(a.ctile_pre[s]))) * a.cell_tile, ldc(ldc(S.mut)->ncell));
+    }
+    stats_flush(a, st);
+}
+
+// One launch: a tile's links, then its joins. Other waves' links may still be
+// on their way when a wave compares roots; it then tests a pair that a later
+// look would have found joined.
+template <class ST>
+__global__ __launch_bounds__(64 * kCellWaves) void k_merge_cells(BatchArgs a) {
+    __shared__ int2 links[kCellWaves][kLinkCap];
+    __shared__ uint32_t pairs[kCellWaves][kPairCap], rest[kCellWaves][kPairCap];
+    const int wv = threadIdx.x >> 6;
+    ST st;
+    LinkBuf lb{links[wv], 0};
+    PairBuf pb{pairs[wv], 0}, far{rest[wv], 0};
+    each_cell_tile(a, st, [&](const StreamDev &S, const CellView &V, int c0, int ncell) {
+        const int k = ldc(S.k), T = a.cell_tile;
+        if (V.dim == 3) link_tile<3>(V, k, c0, T, ncell, lb, st);
+        else if (V.dim == 2) link_tile<2>(V, k, c0, T, ncell, lb, st);
+        else link_tile<1>(V, k, c0, T, ncell, lb, st);
+        join_tile(V, k, c0, T, ncell, pb, far, st);
+    });
 }
 
 // Range count, point-parallel form (large batches, where the device is
@@ -2104,7 +2400,7 @@ __device__ __forceinline__ void count_vblock(const BatchArgs &a, const QueryLane
     const bool valid = p < ql.x.p1;
     const int minpts = V.min_pts;
     int cnt = 0;
-    bool dense = false;
+    bool dense = false, safe = true;
     int c = 0;
     // the query's cell and coordinates, one round trip
     const uint32_t po = (uint32_t)(valid ? p : ql.x.p0) << 2;
@@ -2117,7 +2413,9 @@ __device__ __forceinline__ void count_vblock(const BatchArgs &a, const QueryLane
     arrived(qz);
     if (valid) {
         c = cv;
-        dense = V.cflag[c] & kCellDense;
+        const int cf = V.cflag[c];
+        dense = cf & kCellDense;
+        safe = cf & kCellSafe;
     }
     int tests = 0;
     if (valid && !dense) cnt = count_walk<D>(V, c, qx, qy, qz, ql.sub, LPQ, tests);
@@ -2133,7 +2431,10 @@ __device__ __forceinline__ void count_vblock(const BatchArgs &a, const QueryLane
         }
     }
     cnt = group_sum<LPQ>(cnt);
-    if (valid && ql.sub == 0) V.flags[p] = dense ? (kFlagCore | kFlagDense) : (cnt >= minpts ? kFlagCore : 0);
+    if (valid && ql.sub == 0) {
+        V.flags[p] = dense ? (kFlagCore | kFlagDense) : (cnt >= minpts ? kFlagCore : 0);
+        if (!safe) V.uf[V.W + p] = ufe(vslot(V, p), V.W + p);  // a core of an unsafe cell is an element
+    }
 }
 
 template <int LPQ>
@@ -2158,8 +2459,8 @@ __global__ __launch_bounds__(64) void k_count_points(BatchArgs a) {
 // early exit: the minimum root of the cores within eps. A candidate's flags
 // and element load only when it is within eps.
 template <int D>
-__device__ __forceinline__ int border_walk(const CellView &V, const int32_t *parent, int c, float qx, float qy,
-                                           float qz, int first, int step, int &tests) {
+__device__ __forceinline__ int border_walk(const CellView &V, int c, float qx, float qy, float qz, int first,
+                                           int step, int &tests) {
     const float e2 = V.eps2;
     int best = INT_MAX;
     for (int r0 = first; r0 < V.R; r0 += kBorderRows * step) {
@@ -2194,7 +2495,7 @@ __device__ __forceinline__ int border_walk(const CellView &V, const int32_t *par
             for (int u = 0; u < kFlat; u++)
                 if ((u < nv) & (sqd(D, qx, qy, qz, cx[u], cy[u], cz[u]) < e2) &&
                     (ldo(V.flags, (uint32_t)pos[u]) & kFlagCore))
-                    best = min(best, uf_root(parent, ldo(V.rep, (uint32_t)pos[u] << 2)));
+                    best = min(best, core_cid(V, V.uf[ldo(V.pcell, (uint32_t)pos[u] << 2)], pos[u]));
         }
     }
     return best;
@@ -2213,14 +2514,11 @@ __device__ __forceinline__ void border_vblock(const BatchArgs &a, const QueryLan
     const float qy = D > 1 ? ldo(V.sy, po) : 0.f;
     const float qz = D > 2 ? ldo(V.sz, po) : 0.f;
     const uint64_t qk = ldo(V.skey, po << 1);
-    const int qr = ldo(V.rep, po);
     arrived(c);
     arrived(qx);
     arrived(qy);
     arrived(qz);
     arrived(qk);
-    arrived(qr);
-    const int32_t *parent = ldc(a.s[s].parent);
     const IO io = a.use_io1 ? a.io1 : a.io[s];
     if (vb == ldc(a.pre_chunk[s]) * LPQ && lane_id() == 0) {  // the stream's first block
         StreamMut *m = ldc(a.s[s].mut);
@@ -2231,12 +2529,12 @@ __device__ __forceinline__ void border_vblock(const BatchArgs &a, const QueryLan
     if (p < ql.x.p1 && (qf & kFlagCore) && ql.sub == 0) {
         const int slot = (int)((uint32_t)qk & V.smask);
         gl(io.label)[slot] = 0;
-        gl(io.cid)[slot] = uf_root(parent, qr);
+        gl(io.cid)[slot] = core_cid(V, V.uf[c], pp);
     }
     const bool mine = p < ql.x.p1 && !(qf & kFlagCore);
     int best = INT_MAX;
     int tests = 0;
-    if (mine) best = border_walk<D>(V, parent, c, qx, qy, qz, ql.sub, LPQ, tests);
+    if (mine) best = border_walk<D>(V, c, qx, qy, qz, ql.sub, LPQ, tests);
     if (a.stats) {
         const unsigned long long t = (unsigned long long)wave_sum(tests);
         if (lane_id() == 0 && t) atomicAdd(a.stats + (size_t)s * kNumStats + kStatBorderTests, t);
@@ -2289,14 +2587,11 @@ __device__ __forceinline__ void border_chunk(const BatchArgs &a, const ChunkCtx 
     const float qy = D > 1 ? ldo(V.sy, po) : 0.f;
     const float qz = D > 2 ? ldo(V.sz, po) : 0.f;
     const uint64_t qk = ldo(V.skey, po << 1);
-    const int qr = ldo(V.rep, po);
     arrived(c);
     arrived(qx);
     arrived(qy);
     arrived(qz);
     arrived(qk);
-    arrived(qr);
-    const int32_t *parent = ldc(a.s[s].parent);
     const IO io = a.use_io1 ? a.io1 : a.io[s];
     if (g == ldc(a.pre_chunk[s]) && lane == 0) {  // the stream's first block
         StreamMut *m = ldc(a.s[s].mut);
@@ -2308,7 +2603,7 @@ __device__ __forceinline__ void border_chunk(const BatchArgs &a, const ChunkCtx 
     const bool core = valid && (qf & kFlagCore);
     if (core) {
         gl(io.label)[slot] = 0;
-        gl(io.cid)[slot] = uf_root(parent, qr);
+        gl(io.cid)[slot] = core_cid(V, V.uf[c], pp);
     }
     const uint64_t nm = __ballot(valid && !core);
     if (valid && !core) lq[__popcll(nm & ((1ull << lane) - 1ull))] = BorderQ{c, qx, qy, qz, slot};
@@ -2323,7 +2618,7 @@ __device__ __forceinline__ void border_chunk(const BatchArgs &a, const ChunkCtx 
         const bool have = i < nn;
         const BorderQ q = lq[have ? i : 0];
         int best = INT_MAX;
-        if (have) best = border_walk<D>(V, parent, q.c, q.x, q.y, q.z, sub, 4, tests);
+        if (have) best = border_walk<D>(V, q.c, q.x, q.y, q.z, sub, 4, tests);
         best = group_min<4>(best);
         if (have && sub == 0) {
             gl(io.label)[q.slot] = best != INT_MAX ? 1 : 2;
@@ -2347,488 +2642,35 @@ __global__ __launch_bounds__(64) void k_border_regroup(BatchArgs a) {
     else border_chunk<1>(a, x, g, s, V, lq);
 }
 
-// First core of every cell and union-find element of every position, in one
-// pass after the point-parallel count: one thread per position, a wave on 64
-// consecutive positions. Positions within a cell are in slot order, so a
-// cell's first core is its minimum-slot core: the lowest core flag of the
-// wave's ballot within the cell's lanes when the cell starts in this wave,
-// otherwise (it starts in an earlier wave, or holds no core in this one and
-// runs past it) a scan of its flags. The thread at the cell's first position
-// records fcore.
-__global__ __launch_bounds__(kTileThreads) void k_fcore_rep(BatchArgs a) {
-    const int g = blockIdx.x;
-    const int s = find_stream_c(a.pre_wtile, a.n, g);
-    const StreamDev &S = a.s[s];
-    const int W = ldc(S.W);
+// First core and union-find entry of every cell, after the point-parallel
+// count: one lane per cell. Positions within a cell are in slot order, so the
+// first core has the cell's minimum core slot. A dense cell's is its first
+// point, and the others' flags are few (fewer than min_pts points, reach 1
+// apart), read four at a time.
+__global__ __launch_bounds__(64 * kCellWaves) void k_cell_cores(BatchArgs a) {
+    const int total = uni(ldc(a.ctile_pre[a.n]));
     const int lane = lane_id();
-    const int p0 = (g - ldc(a.pre_wtile[s])) * kWTile;
+    int s = 0;
+    for (int g = uni(blockIdx.x * kCellWaves + (threadIdx.x >> 6)); g < total; g += gridDim.x * kCellWaves) {
+        s = uni(find_stream_from(a.ctile_pre, a.n, g, s));
+        const StreamDev &S = a.s[s];
+        const CellView V = cell_view(S);
+        const int c = (g - uni(ldc(a.ctile_pre[s]))) * a.cell_tile + lane;
+        if (lane >= a.cell_tile || c >= ldc(ldc(S.mut)->ncell)) continue;
+        const int cf = V.cflag[c], cs = V.cstart[c], ce = V.cstart[c + 1];
+        int fc = (cf & kCellDense) ? cs : kNoCore;
+        for (int i = cs; i < ce && fc == kNoCore; i += 4) {
+            int f[4];
 #pragma unroll
-    for (int r = 0; r < kWTile / kTileThreads; r++) {
-        const int p = p0 + r * kTileThreads + threadIdx.x;
-        const int wb = p - lane;  // the wave's first position
-        // a wave past the window's end (the last tile's tail) has no position;
-        // in the others the lanes past the end read the wave's first position
-        if (wb >= W) break;
-        const bool v = p < W;
-        const int pp = v ? p : wb;
-        const int c = S.pcell[pp];
-        const int f = S.flags[pp];
-        const int cf = S.cflag[c];
-        const int cs = S.cstart[c], ce = S.cstart[c + 1];
-        const uint64_t corem = __ballot(v && (f & kFlagCore));
-        int fc = kNoCore;
-        if (cf & kCellDense) {
-            fc = cs;
-        } else {
-            int from = cs;  // positions still to scan: [from, ce)
-            if (cs >= wb) {
-                const int lo = cs - wb, hi = min(ce - wb, 64);
-                const uint64_t m = corem & (~0ull << lo) & (hi >= 64 ? ~0ull : ((1ull << hi) - 1ull));
-                if (m) fc = wb + __ffsll((unsigned long long)m) - 1;
-                from = m ? ce : wb + 64;
-            }
-            for (int i = from; i < ce; i++)
-                if (S.flags[i] & kFlagCore) {
-                    fc = i;
-                    break;
-                }
+            for (int q = 0; q < 4; q++) f[q] = V.flags[min(i + q, ce - 1)];
+#pragma unroll
+            for (int q = 3; q >= 0; q--)
+                if ((f[q] & kFlagCore) && i + q < ce) fc = i + q;
         }
-        if (v && p == cs) S.fcore[c] = fc;
-        if (v) S.rep[p] = slot_of(S, (cf & kCellSafe) && fc != kNoCore ? fc : p);
+        V.fcore[c] = fc;
+        V.uf[c] = fc == kNoCore ? kUfNone : ((cf & kCellSafe) ? ufe(vslot(V, fc), c) : kUfUnsafe);
     }
 }
-
-// Cluster merge, cell level, for safe cells: all cores of a safe cell belong
-// to one cluster (its points are within eps of each other), so two safe cells
-// join as soon as one core pair is within eps - the analogue of the
-// reference's dense-cell spheres, where a ray unites with the first point of
-// the cell within eps and stops (dbscan.cu:378-393). Only stencil cells
-// B < A are tested, so each unordered pair of cells is tested once.
-//
-// A wave serves kUGCells query cells per round. Each query cell's cores are
-// staged in LDS; the stencil rows of all the round's cells are spread over the
-// lanes, their candidate cells are concatenated into one list, and each lane
-// tests one (query cell, candidate) pair at a time. Touching pairs go to an
-// LDS edge list that the lanes unite together at the end of the round, so a
-// round costs a few dependent memory round trips for all its cells. Pairs
-// needing more than kUGWork point tests are queued and tested by the whole wave;
-// query cells with more than kUGCap cores are served by the whole wave
-// (union_cell_wave).
-constexpr int kUG = 64 / kUGCells;            // lanes staging one query cell
-constexpr int kUGCap = 64;                    // cores of a query cell staged in LDS
-constexpr int kUGWork = 256;                  // larger pair tests (cores x points): whole wave
-constexpr int kUGQueue = 128;                 // queued (query cell, candidate) pairs
-constexpr int kUGRows = kUGCells * kMaxRows;  // stencil rows of one round
-constexpr int kUGEdges = 256;                 // buffered touching pairs
-constexpr int kUnionA = kUGCells * kUGCap;    // LDS capacity for a large query cell
-constexpr int kUnionB = 8;                    // register capacity for a candidate cell
-
-struct UnionLds {
-    float x[kUGCells * kUGCap], y[kUGCells * kUGCap], z[kUGCells * kUGCap];
-    uint8_t lc[kUnionA];       // whole-wave path: core flags of the query cell
-    int ncore[kUGCells];       // cores staged for the group's cell
-    int rep[kUGCells];         // representative slot of the group's cell
-    int sidx[kUGCells];        // stream of the group's cell
-    int cell[kUGCells];        // the group's cell (stream-local)
-    int mode[kUGCells];        // 0 idle, 1 staged, 2 whole-wave path
-    int rowbase[kUGCells + 1]; // first row of each group in the round's row list
-    int rowpre[kUGRows + 1];   // exclusive prefix of candidate counts
-    int rowclo[kUGRows];       // first candidate cell of the row
-    int2 q[kUGQueue];          // (group, candidate cell)
-    int2 edge[kUGEdges];       // (group, representative slot of the candidate)
-    int nq;
-};
-
-__device__ __forceinline__ void flush_edges(const BatchArgs &a, UnionLds &L, int &ne) {
-    for (int i = lane_id(); i < ne; i += 64) {
-        const int2 e = L.edge[i];
-        uf_unite(a.s[L.sidx[e.x]].parent, L.rep[e.x], e.y);
-    }
-    ne = 0;
-}
-
-// Appends the touching pairs of the wave (lanes with want set) to the edge
-// list, in lane order; all lanes call it together.
-__device__ __forceinline__ void push_edges(const BatchArgs &a, UnionLds &L, int &ne, bool want, int g, int v) {
-    const uint64_t m = __ballot(want);
-    if (m == 0ull) return;
-    const int n = __popcll(m);
-    if (ne + n > kUGEdges) {
-        __syncthreads();
-        flush_edges(a, L, ne);
-        __syncthreads();
-    }
-    if (want) L.edge[ne + __popcll(m & ((1ull << lane_id()) - 1ull))] = make_int2(g, v);
-    ne += n;
-}
-
-// Whole-wave test of one (query cell, large candidate cell B) pair: lanes
-// over B's points, a loop over the query cell's staged cores, stop at the
-// first pair within eps.
-__device__ void union_pair_wave(const StreamDev &S, const float *qx, const float *qy, const float *qz, int ncore,
-                                int rep, int B) {
-    const int lane = lane_id(), dim = S.dim;
-    const float e2 = S.eps2;
-    const uint8_t cfB = S.cflag[B];
-    const int fcB = S.fcore[B];
-    const int csB = S.cstart[B], ceB = S.cstart[B + 1];
-    bool touch = false;
-    for (int b0 = csB; b0 < ceB && !touch; b0 += 64) {
-        const int pb = b0 + lane;
-        bool vb = pb < ceB;
-        float bx = 0.f, by = 0.f, bz = 0.f;
-        if (vb) {
-            vb = (cfB & kCellDense) || (S.flags[pb] & kFlagCore);
-            bx = S.sx[pb];
-            if (dim > 1) by = S.sy[pb];
-            if (dim > 2) bz = S.sz[pb];
-        }
-        for (int i = 0; i < ncore; i++) {
-            if (__ballot(vb && sqd(dim, qx[i], qy[i], qz[i], bx, by, bz) < e2) != 0ull) {
-                touch = true;
-                break;
-            }
-        }
-    }
-    if (touch && lane == 0) uf_unite(S.parent, rep, slot_of(S, fcB));
-}
-
-// Whole-wave merge of one large safe query cell A with its stencil cells
-// B < A: lanes take candidate cells; A's points sit in LDS when they fit,
-// and a small B is held in the lane's registers.
-__device__ void union_cell_wave(const StreamDev &S, int A, UnionLds &L) {
-    const int lane = lane_id();
-    const uint8_t cfA = S.cflag[A];
-    const int fcA = S.fcore[A];
-    const int dim = S.dim;
-    const float e2 = S.eps2;
-    float *lx = L.x, *ly = L.y, *lz = L.z;
-    // stencil cells B < A, row by row: [pcell[rb], min(pcell[re-1], A-1)]
-    int clo = 0, cnt = 0;
-    if (lane < S.R) {
-        const int2 r = S.rows[(size_t)A * S.R + lane];
-        if (r.x < r.y) {
-            clo = S.pcell[r.x];
-            const int chi = min(S.pcell[r.y - 1], A - 1);
-            cnt = max(0, chi - clo + 1);
-        }
-    }
-    int incl = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-    }
-    const int pre = incl - cnt;
-    const int TC = __shfl(incl, 63);
-    if (TC == 0) return;
-    const int csA = S.cstart[A], ceA = S.cstart[A + 1], nA = ceA - csA;
-    const bool inl = nA <= kUnionA;
-    const int sA = slot_of(S, fcA);
-    __syncthreads();
-    if (inl) {
-        for (int i = lane; i < nA; i += 64) {
-            lx[i] = S.sx[csA + i];
-            ly[i] = dim > 1 ? S.sy[csA + i] : 0.f;
-            lz[i] = dim > 2 ? S.sz[csA + i] : 0.f;
-            L.lc[i] = (cfA & kCellDense) ? (uint8_t)1 : (uint8_t)(S.flags[csA + i] & kFlagCore);
-        }
-    }
-    __syncthreads();
-    for (int jb = 0; jb < TC; jb += 64) {
-        const int j = jb + lane;
-        const int jj = j < TC ? j : TC - 1;
-        const int r = row_of(pre, S.R, jj);
-        const int B = __shfl(clo, r) + (jj - __shfl(pre, r));
-        bool big = false;
-        bool touch = false;
-        int fcB = kNoCore;
-        if (j < TC) {
-            const uint8_t cfB = S.cflag[B];
-            fcB = S.fcore[B];
-            if ((cfB & kCellSafe) && fcB != kNoCore) {
-                const int csB = S.cstart[B], nB = S.cstart[B + 1] - csB;
-                if (inl && nB <= kUnionB) {
-                    float bx[kUnionB], by[kUnionB], bz[kUnionB];
-                    bool bc[kUnionB];
-#pragma unroll
-                    for (int m = 0; m < kUnionB; m++) {
-                        bc[m] = false;
-                        bx[m] = by[m] = bz[m] = 0.f;
-                        if (m < nB) {
-                            bc[m] = (cfB & kCellDense) || (S.flags[csB + m] & kFlagCore);
-                            bx[m] = S.sx[csB + m];
-                            if (dim > 1) by[m] = S.sy[csB + m];
-                            if (dim > 2) bz[m] = S.sz[csB + m];
-                        }
-                    }
-                    for (int i = 0; i < nA && !touch; i++) {
-                        if (!L.lc[i]) continue;
-                        const float qx = lx[i], qy = ly[i], qz = lz[i];
-#pragma unroll
-                        for (int m = 0; m < kUnionB; m++)
-                            touch = touch || (bc[m] && sqd(dim, qx, qy, qz, bx[m], by[m], bz[m]) < e2);
-                    }
-                } else {
-                    big = true;
-                }
-            }
-        }
-        if (touch) uf_unite(S.parent, sA, slot_of(S, fcB));
-        // large candidate cells of this batch: one at a time, lanes over B's
-        // points, a loop over A's cores, stop at the first pair within eps
-        uint64_t bigm = __ballot(big);
-        while (bigm) {
-            const int l = __ffsll((unsigned long long)bigm) - 1;
-            bigm &= bigm - 1;
-            const int Bl = lane_i(B, l);
-            const uint8_t cfB = S.cflag[Bl];
-            const int fcBl = S.fcore[Bl];
-            const int csB = S.cstart[Bl], ceB = S.cstart[Bl + 1];
-            bool t = false;
-            for (int b0 = csB; b0 < ceB && !t; b0 += 64) {
-                const int pb = b0 + lane;
-                bool vb = pb < ceB;
-                float bx = 0.f, by = 0.f, bz = 0.f;
-                if (vb) {
-                    vb = (cfB & kCellDense) || (S.flags[pb] & kFlagCore);
-                    bx = S.sx[pb];
-                    if (dim > 1) by = S.sy[pb];
-                    if (dim > 2) bz = S.sz[pb];
-                }
-                for (int i = 0; i < nA; i++) {
-                    float qx, qy, qz;
-                    bool qc;
-                    if (inl) {
-                        qc = L.lc[i];
-                        qx = lx[i];
-                        qy = ly[i];
-                        qz = lz[i];
-                    } else {
-                        qc = (cfA & kCellDense) || (S.flags[csA + i] & kFlagCore);
-                        qx = S.sx[csA + i];
-                        qy = dim > 1 ? S.sy[csA + i] : 0.f;
-                        qz = dim > 2 ? S.sz[csA + i] : 0.f;
-                    }
-                    if (!qc) continue;
-                    if (__ballot(vb && sqd(dim, qx, qy, qz, bx, by, bz) < e2) != 0ull) {
-                        t = true;
-                        break;
-                    }
-                }
-            }
-            if (t && lane == 0) uf_unite(S.parent, sA, slot_of(S, fcBl));
-        }
-    }
-}
-
-__global__ __launch_bounds__(64) void k_union_cells(BatchArgs a) {
-    __shared__ UnionLds L;
-    const int lane = lane_id(), grp = lane / kUG, sub = lane % kUG;
-    const uint64_t gmask = ((1ull << kUG) - 1ull) << (grp * kUG);
-    const int total = ldc(a.cell_pre[a.n]);
-    // Round r of wave b serves cells b + (r * kUGCells + g) * gridDim.x: the
-    // cells of a round are far apart, so dense regions (long pair tests) are
-    // spread over many waves instead of falling to a few.
-    const int G = gridDim.x;
-    for (int base = 0; base + (int)blockIdx.x < total; base += G * kUGCells) {
-        // 1. stage each group's query cell: its cores, compacted, in LDS
-        const int gc = (int)blockIdx.x + base + grp * G;
-        int mode = 0, ncore = 0, A = 0, sidx = 0, rep = 0, R = 0;
-        if (gc < total) {
-            const CellCtx x = cell_of(a, gc);
-            sidx = x.s;
-            A = x.c;
-            const StreamDev &S = a.s[sidx];
-            const uint8_t cfA = S.cflag[A];
-            const int fcA = S.fcore[A];
-            if ((cfA & kCellSafe) && fcA != kNoCore) {
-                const int csA = S.cstart[A], nA = S.cstart[A + 1] - csA;
-                const bool denseA = cfA & kCellDense;
-                const int dim = S.dim;
-                float *gx = L.x + grp * kUGCap, *gy = L.y + grp * kUGCap, *gz = L.z + grp * kUGCap;
-                rep = slot_of(S, fcA);
-                for (int i0 = 0; i0 < nA; i0 += kUG) {
-                    const int i = i0 + sub;
-                    bool c = false;
-                    float px = 0.f, py = 0.f, pz = 0.f;
-                    if (i < nA) {
-                        c = denseA || (S.flags[csA + i] & kFlagCore);
-                        px = S.sx[csA + i];
-                        if (dim > 1) py = S.sy[csA + i];
-                        if (dim > 2) pz = S.sz[csA + i];
-                    }
-                    const uint64_t m = __ballot(c) & gmask;
-                    const int pos = ncore + __popcll(m & ((1ull << lane) - 1ull));
-                    if (c && pos < kUGCap) {
-                        gx[pos] = px;
-                        gy[pos] = py;
-                        gz[pos] = pz;
-                    }
-                    ncore += __popcll(m);
-                }
-                mode = ncore <= kUGCap ? 1 : 2;
-                R = mode == 1 ? S.R : 0;
-            }
-        }
-        if (sub == 0) {
-            L.mode[grp] = mode;
-            L.ncore[grp] = ncore;
-            L.rep[grp] = rep;
-            L.sidx[grp] = sidx;
-            L.cell[grp] = A;
-        }
-        // rows of group g occupy [rbase[g], rbase[g+1]) of the round's row list
-        int rbase[kUGCells + 1];
-        rbase[0] = 0;
-#pragma unroll
-        for (int g = 0; g < kUGCells; g++) rbase[g + 1] = rbase[g] + __shfl(R, g * kUG);
-        if (lane <= kUGCells) {
-            int v = 0;
-#pragma unroll
-            for (int g = 0; g <= kUGCells; g++) v = lane == g ? rbase[g] : v;
-            L.rowbase[lane] = v;
-        }
-        const int NR = rbase[kUGCells];
-        __syncthreads();
-        // 2. rows of all groups over the lanes: candidate cells B < A per row
-        int run = 0;
-        for (int t0 = 0; t0 < NR; t0 += 64) {
-            const int t = t0 + lane;
-            int cnt = 0, clo = 0;
-            if (t < NR) {
-                int g = 0;
-#pragma unroll
-                for (int h = 1; h < kUGCells; h++) g += t >= rbase[h];
-                const StreamDev &S = a.s[L.sidx[g]];
-                const int Ag = L.cell[g];
-                const int2 rr = S.rows[(size_t)Ag * S.R + (t - L.rowbase[g])];
-                if (rr.x < rr.y) {
-                    clo = S.pcell[rr.x];
-                    const int chi = min(S.pcell[rr.y - 1], Ag - 1);
-                    cnt = max(0, chi - clo + 1);
-                }
-                L.rowclo[t] = clo;
-            }
-            int incl = cnt;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int y = __shfl_up(incl, o);
-                if (lane >= o) incl += y;
-            }
-            if (t < NR) L.rowpre[t] = run + incl - cnt;
-            run += __shfl(incl, 63);
-        }
-        const int TC = run;
-        if (lane == 0) {
-            L.rowpre[NR] = TC;
-            L.nq = 0;
-        }
-        __syncthreads();
-        // 3. (query cell, candidate) pairs over the lanes
-        int ne = 0;
-        for (int jb = 0; jb < TC; jb += 64) {
-            const int j = jb + lane;
-            bool touch = false;
-            int g = 0, vrep = 0;
-            if (j < TC) {
-                int lo = 0, hi = NR;  // last row t with rowpre[t] <= j
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (L.rowpre[mid] <= j) lo = mid;
-                    else hi = mid;
-                }
-                const int t = lo;
-#pragma unroll
-                for (int h = 1; h < kUGCells; h++) g += t >= rbase[h];
-                const int B = L.rowclo[t] + (j - L.rowpre[t]);
-                const StreamDev &S = a.s[L.sidx[g]];
-                const uint8_t cfB = S.cflag[B];
-                const int fcB = S.fcore[B];
-                if ((cfB & kCellSafe) && fcB != kNoCore) {
-                    const int csB = S.cstart[B], nB = S.cstart[B + 1] - csB;
-                    bool queued = false;
-                    if (L.ncore[g] * nB > kUGWork) {
-                        const int e = atomicAdd(&L.nq, 1);
-                        if (e < kUGQueue) {
-                            L.q[e] = make_int2(g, B);
-                            queued = true;
-                        }
-                    }
-                    if (!queued) {
-                        const int dim = S.dim, nc = L.ncore[g];
-                        const float e2 = S.eps2;
-                        const float *qx = L.x + g * kUGCap, *qy = L.y + g * kUGCap, *qz = L.z + g * kUGCap;
-                        const bool denseB = cfB & kCellDense;
-                        for (int b0 = 0; b0 < nB && !touch; b0 += 4) {
-                            float bx[4], by[4], bz[4];
-                            bool bc[4];
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                const int jj = csB + min(b0 + u, nB - 1);
-                                bc[u] = (b0 + u < nB) && (denseB || (S.flags[jj] & kFlagCore));
-                                bx[u] = S.sx[jj];
-                                by[u] = dim > 1 ? S.sy[jj] : 0.f;
-                                bz[u] = dim > 2 ? S.sz[jj] : 0.f;
-                            }
-                            for (int i = 0; i < nc && !touch; i++) {
-                                const float ax = qx[i], ay = qy[i], az = qz[i];
-#pragma unroll
-                                for (int u = 0; u < 4; u++)
-                                    touch = touch || (bc[u] && sqd(dim, ax, ay, az, bx[u], by[u], bz[u]) < e2);
-                            }
-                        }
-                        if (touch) vrep = slot_of(S, fcB);
-                    }
-                }
-            }
-            push_edges(a, L, ne, touch, g, vrep);
-        }
-        __syncthreads();
-        flush_edges(a, L, ne);
-        __syncthreads();
-        // 4. queued large candidate cells, then large query cells: whole wave
-        const int nq = min(L.nq, kUGQueue);
-        for (int e = 0; e < nq; e++) {
-            const int2 it = L.q[e];
-            const int g = it.x;
-            union_pair_wave(a.s[L.sidx[g]], L.x + g * kUGCap, L.y + g * kUGCap, L.z + g * kUGCap, L.ncore[g],
-                            L.rep[g], it.y);
-        }
-        for (int g = 0; g < kUGCells; g++) {
-            if (L.mode[g] != 2) continue;
-            union_cell_wave(a.s[L.sidx[g]], L.cell[g], L);
-        }
-        __syncthreads();  // the next round overwrites the LDS
-    }
-}
-
-// Cluster merge, point level, for the cores of unsafe cells (grid border, or
-// grids whose cells are not dense-safe): each unites with every core within
-// eps (the reference's core branch of __intersection__hybrid_radius_sphere,
-// dbscan.cu:364-369), through the representatives of safe cells.
-__device__ __forceinline__ void union_points_chunk(const BatchArgs &a, int g) {
-    const ChunkCtx x = chunk_of(a, g);
-    const StreamDev &S = a.s[x.s];
-    const int p = x.p0 + lane_id();
-    if (p >= x.p1) return;
-    if (!(S.flags[p] & kFlagCore)) return;
-    const int c = S.pcell[p];
-    if (S.cflag[c] & kCellSafe) return;  // k_union_cells
-    const int dim = S.dim;
-    const float e2 = S.eps2;
-    const float qx = S.sx[p];
-    const float qy = dim > 1 ? S.sy[p] : 0.f;
-    const float qz = dim > 2 ? S.sz[p] : 0.f;
-    const int sp = slot_of(S, p);
-    walk_candidates(cell_view(S), c, [&](int j, float cx, float cy, float cz) {
-        if (j != p && sqd(dim, qx, qy, qz, cx, cy, cz) < e2 && (S.flags[j] & kFlagCore))
-            uf_unite(S.parent, sp, rep_slot(S, j));
-        return false;
-    });
-}
-
-__global__ __launch_bounds__(64) void k_union_points(BatchArgs a) { union_points_chunk(a, blockIdx.x); }
 
 // Plain device copy of 16-byte words: a kernel of known HBM traffic (reads and
 // writes `n16` * 16 bytes) used to scale the profiler's byte counters.
@@ -2894,7 +2736,7 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
     RTDBS_LAUNCH(k_cells, sh.wtiles, kTileThreads, a);
     PH_END(kPhCells);
     PH_BEGIN(kPhRows);
-    RTDBS_LAUNCH(k_rows, sh.rows_blocks, kTileThreads, a);
+    RTDBS_LAUNCH(k_rows, sh.rows_blocks + 1, kTileThreads, a);
     PH_END(kPhRows);
     {
         // The range-count kernel is timed by its own dispatch: the events take
@@ -2912,18 +2754,13 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
         if (e != hipSuccess) return e;
     }
     PH_BEGIN(kPhUnion);
-    // the cell-parallel count wrote every cell's first core and every
-    // position's union-find element; after the point-parallel count one pass
-    // over the positions does
-    if (!sh.count_cell) RTDBS_LAUNCH(k_fcore_rep, sh.wtiles, kTileThreads, a);
-    if (sh.union_cells) {
-        RTDBS_LAUNCH(k_union_cells, sh.cell_blocks, 64, a);
-        RTDBS_LAUNCH(k_union_points, sh.chunks, 64, a);
-    } else if (a.stats) {
-        RTDBS_LAUNCH(k_union<WaveStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
-    } else {
-        RTDBS_LAUNCH(k_union<NoStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
-    }
+    // the cell-parallel count wrote every cell's first core and entry; after
+    // the point-parallel count a pass over the cells does
+    if (!sh.count_cell) RTDBS_LAUNCH(k_cell_cores, sh.link_blocks, 64 * kCellWaves, a);
+    if (sh.link && a.stats) RTDBS_LAUNCH(k_merge_cells<WaveStats>, sh.link_blocks, 64 * kCellWaves, a);
+    else if (sh.link) RTDBS_LAUNCH(k_merge_cells<NoStats>, sh.link_blocks, 64 * kCellWaves, a);
+    if (sh.unsafe && a.stats) RTDBS_LAUNCH(k_union<WaveStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
+    else if (sh.unsafe) RTDBS_LAUNCH(k_union<NoStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
     PH_END(kPhUnion);
     PH_BEGIN(kPhBorder);
     if (sh.cellpar && a.stats) RTDBS_LAUNCH(k_border<WaveStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
