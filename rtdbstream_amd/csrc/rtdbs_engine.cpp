@@ -592,9 +592,11 @@ static int env_int(const char *name, int def, int lo, int hi) {
     return (x >= lo && x <= hi) ? x : def;
 }
 
-// Windows up to this many points in one launch use the cell-parallel count
-// and border kernels.
+// Windows up to this many points in one launch use the cell-parallel count of
+// a single stream, and the launch sizes of a latency-bound launch.
 constexpr long long kCellParMaxPoints = 1000000;
+// The same for the cell-parallel outputs, and the count of several streams.
+constexpr long long kCellParMaxShared = 250000;
 
 // Uploads descriptors and prefix tables; drops a captured graph. Called when
 // the batch is built and whenever a member stream was re-initialised.
@@ -644,19 +646,26 @@ int refresh_batch(rtdbs_batch *b) {
     const int r_def = p1 && p1->rows_per_cu > 0 ? p1->rows_per_cu : (cells_total <= kCellParMaxPoints ? 8 : 32);
     const int rcap = env_int("RTDBS_ROWS_PER_CU", r_def, 1, kMaxPerCu);
     b->shape.rows_blocks = (int)std::max(1ll, std::min((long long)device_cus() * rcap, pb));
-    // Count and border: cell-parallel (coalesced candidate loads, more
-    // instructions per query) while a launch is small and latency-bound,
-    // point-parallel once its total window saturates the device.
+    // Count and outputs: cell-parallel (coalesced candidate loads, a wave per
+    // cell) while a launch is small and latency-bound, point-parallel once its
+    // windows fill the device's lanes. A batch of several streams switches both
+    // above kCellParMaxShared points (us cell / point: 338,000 points of 16
+    // streams count 56 / 50, outputs 58 / 46; 687,000 of 32 streams 89 / 62, 103 /
+    // 60; 110,000 of 8 streams 23 / 19, 24 / 38). A single stream's outputs switch
+    // there too (500,000 3-D points 53 / 43, 1-D 33 / 12; 100,000 13 / 18), its
+    // count only above kCellParMaxPoints (500,000 points 45 / 73, 1 M 121 / 183).
     // RTDBS_NEIGHBOR_MODE: 1 forces cell-parallel, 2 point-parallel (over a
     // single stream's own neighbor_mode).
     const int nmode = env_int("RTDBS_NEIGHBOR_MODE", 0, 0, 2);
     const int pmode = n == 1 ? b->streams[0]->p.neighbor_mode : 0;  // a single stream's own setting
     const int mode = nmode ? nmode : pmode;
-    b->shape.cellpar = mode == 1 || (mode == 0 && cells_total <= kCellParMaxPoints);
+    b->shape.cellpar = mode == 1 || (mode == 0 && cells_total <= kCellParMaxShared);
     // the range count's own form (RTDBS_COUNT_MODE: 1 cell-parallel, 2
-    // point-parallel; otherwise as the output kernel)
+    // point-parallel; otherwise as above)
     const int cmode = env_int("RTDBS_COUNT_MODE", 0, 0, 2);
-    b->shape.count_cell = cmode ? (cmode == 1) : b->shape.cellpar;
+    b->shape.count_cell =
+        cmode ? (cmode == 1)
+              : mode == 1 || (mode == 0 && cells_total <= (n == 1 ? kCellParMaxPoints : kCellParMaxShared));
     // cell-parallel grid: 16 blocks per CU while the launch is small; 32 for
     // large batches, where it carries the merge alone (64 streams: 455 ->
     // ~400 us). RTDBS_CELLPAR_PER_CU overrides.
@@ -670,11 +679,14 @@ int refresh_batch(rtdbs_batch *b) {
     b->shape.link = b->shape.unsafe = 0;
     for (int i = 0; i < n; i++) (b->streams[i]->dense_ok ? b->shape.link : b->shape.unsafe) = 1;
     // Cells per wave of the merge: small tiles keep a latency-bound launch's
-    // waves short (100,000 3-D points: 8 cells 27 us, 64 cells 38), large ones
-    // fill the lanes where waves abound (3.2 M points of 64 streams: 64 cells 138
-    // us, 16 cells 234; 338,000 points of 16 streams: 32 cells best by 2-6%).
-    // RTDBS_CELL_TILE overrides.
-    const int ctile = env_int("RTDBS_CELL_TILE", cells_total <= 200000 ? 8 : (cells_total <= 600000 ? 32 : 64), 1, 64);
+    // waves short, large ones fill the lanes where waves abound. us of the merge
+    // with 8 / 16 / 32 / 64 cells: 100,000 3-D points 27 / 28 / 35 / 38; 110,000
+    // points of 8 streams 28 / 22 / 24 / 31; 338,000 of 16 streams 56 / 41 / 36 /
+    // 40; 1 M points, one stream - / 112 / 90 / 92, 32 streams 155 / 115 / 93 /
+    // 114; 3.2 M of 64 streams - / 234 / 168 / 138. RTDBS_CELL_TILE overrides.
+    const int ctile_def =
+        cells_total <= 100000 ? 8 : (cells_total <= 250000 ? 16 : (cells_total <= 2000000 ? 32 : 64));
+    const int ctile = env_int("RTDBS_CELL_TILE", ctile_def, 1, 64);
     b->shape.link_blocks =
         (int)std::max(1ll, std::min((long long)device_cus() * 16, (cells_total + 4 * ctile - 1) / (4 * ctile)));
     // lanes per query: enough threads to cover the device several times over,
