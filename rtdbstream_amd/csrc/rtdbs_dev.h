@@ -147,6 +147,17 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
                         uint32_t phase_mask);
 // Enqueues the first-window load (sort of W points into the window arrays).
 hipError_t launch_init(const BatchArgs &a, int32_t itiles, int32_t passes, hipStream_t st);
+// One of a list of copies between pinned host memory and the device, of 4-byte
+// words; first: words of the copies before it.
+struct CopySeg {
+    const void *src;
+    void *dst;
+    uint32_t first, words;
+};
+
+// Carries out the n copies of `segs` (memory the device can read), `words` in
+// all, in one launch.
+hipError_t launch_copy_segs(const CopySeg *segs, int n, uint32_t words, hipStream_t st);
 // Copies n16 16-byte words (profiler byte-counter calibration).
 hipError_t launch_copy16(const void *src, void *dst, size_t n16, hipStream_t st);
 

@@ -578,6 +578,7 @@ void batch_free(rtdbs_batch *b) {
     if (b->h_desc) (void)hipHostFree(b->h_desc);
     if (b->h_pre) (void)hipHostFree(b->h_pre);
     if (b->h_stage) (void)hipHostFree(b->h_stage);
+    if (b->h_segs) (void)hipHostFree(b->h_segs);
     if (b->d_xfer) (void)hipFree(b->d_xfer);
     if (b->dmem) (void)hipFree(b->dmem);
     delete b;
@@ -890,6 +891,40 @@ static void add_copy(std::vector<Copy> &v, void *dst, const void *src, size_t by
     v.push_back(Copy{dst, src, bytes});
 }
 
+// The list's slot in the batch's pinned copy lists: `way` 0 up, 1 down, of area p.
+static CopySeg *seg_list(rtdbs_batch *b, int p, int way) {
+    if (!b->h_segs &&
+        hipHostMalloc((void **)&b->h_segs, (size_t)8 * b->capacity * sizeof(CopySeg), hipHostMallocCoherent) !=
+            hipSuccess) {
+        (void)hipGetLastError();
+        b->h_segs = nullptr;
+    }
+    return b->h_segs ? b->h_segs + (size_t)(2 * p + way) * 2 * b->capacity : nullptr;
+}
+
+// Enqueues the copies on st: two or more as one launch over a pinned list
+// (whose previous use on st must have ended), unless a pointer or size is no
+// multiple of 4 bytes.
+static int enqueue_copies(const std::vector<Copy> &v, hipMemcpyKind kind, CopySeg *list, hipStream_t st) {
+    size_t words = 0;
+    bool fit = list && v.size() >= 2;
+    for (const Copy &c : v) {
+        fit = fit && (((uintptr_t)c.dst | (uintptr_t)c.src | c.bytes) & 3) == 0;
+        words += c.bytes / 4;
+    }
+    if (fit && words < (size_t(1) << 32)) {
+        uint32_t first = 0;
+        for (size_t i = 0; i < v.size(); i++) {
+            list[i] = CopySeg{v[i].src, v[i].dst, first, (uint32_t)(v[i].bytes / 4)};
+            first += list[i].words;
+        }
+        HIPCHK(launch_copy_segs(list, (int)v.size(), (uint32_t)words, st));
+        return RTDBS_OK;
+    }
+    for (const Copy &c : v) HIPCHK(hipMemcpyAsync(c.dst, c.src, c.bytes, kind, st));
+    return RTDBS_OK;
+}
+
 // Offsets of every member's stride and outputs in the transfer area and the
 // pinned staging (same layout); (re)allocates both when they are too small.
 static int ensure_xfer(rtdbs_batch *b) {
@@ -968,7 +1003,8 @@ int batch_slide_host(rtdbs_batch *b, const float *const *in, int32_t *const *lab
             add_copy(up, dev, h, nb);
         }
     }
-    for (const Copy &c : up) HIPCHK(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyHostToDevice, b->hs));
+    rc = enqueue_copies(up, hipMemcpyHostToDevice, up.size() > 1 ? seg_list(b, 0, 0) : nullptr, b->hs);
+    if (rc) return rc;
     if (b->solo)
         rc = batch_launch_solo(b, b->stage_io[0].in, b->stage_io[0].label, b->stage_io[0].cid);
     else
@@ -989,7 +1025,8 @@ int batch_slide_host(rtdbs_batch *b, const float *const *in, int32_t *const *lab
             }
         }
     }
-    for (const Copy &c : down) HIPCHK(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, b->hs));
+    rc = enqueue_copies(down, hipMemcpyDeviceToHost, down.size() > 1 ? seg_list(b, 0, 1) : nullptr, b->hs);
+    if (rc) return rc;
     rc = batch_sync(b);
     if (rc) return rc;
     for (const Copy &c : post) std::memcpy(c.dst, c.src, c.bytes);
@@ -1085,7 +1122,8 @@ int batch_slide_pipelined(rtdbs_batch *b, const float *const *in, int32_t *const
         add_copy(down, cids[i], area + b->out_off[i] + nb, nb);
     }
     if (P.issued >= 2) HIPCHK(hipStreamWaitEvent(P.up, P.kern_done[p], 0));
-    for (const Copy &c : up) HIPCHK(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyHostToDevice, P.up));
+    rc = enqueue_copies(up, hipMemcpyHostToDevice, up.size() > 1 ? seg_list(b, p, 0) : nullptr, P.up);
+    if (rc) return rc;
     HIPCHK(hipEventRecord(P.in_done[p], P.up));
     HIPCHK(hipStreamWaitEvent(b->hs, P.in_done[p], 0));
     if (P.issued >= 2) HIPCHK(hipStreamWaitEvent(b->hs, P.out_done[p], 0));
@@ -1112,7 +1150,8 @@ int batch_slide_pipelined(rtdbs_batch *b, const float *const *in, int32_t *const
     }
     HIPCHK(hipEventRecord(P.kern_done[p], b->hs));
     HIPCHK(hipStreamWaitEvent(P.down, P.kern_done[p], 0));
-    for (const Copy &c : down) HIPCHK(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, P.down));
+    rc = enqueue_copies(down, hipMemcpyDeviceToHost, down.size() > 1 ? seg_list(b, p, 1) : nullptr, P.down);
+    if (rc) return rc;
     HIPCHK(hipEventRecord(P.out_done[p], P.down));
     for (auto *s : b->streams) s->slides++;
     if (b->stats_on) b->stats_slides++;

@@ -66,6 +66,10 @@ struct rtdbs_batch {
     char *h_stage = nullptr;
     size_t h_stage_bytes = 0;
     std::vector<size_t> in_off, out_off;
+    // Copy lists of the host-buffer slides, pinned: one of up to 2 * capacity
+    // copies each way, for each of the two areas of the pipelined slides (the
+    // synchronous slide uses the first).
+    rtdbs::CopySeg *h_segs = nullptr;
     // Pipelined host-buffer slides (rtdbs_batch_slide_pipelined): two device
     // areas in the transfer area's layout, used by alternate slides, an I/O
     // table and a captured graph for each, a copy stream each way beside the
