@@ -96,7 +96,6 @@ struct BatchArgs {
     int32_t n;
     const int32_t *pre_stile;  // n+1 prefix of ceil(S/kTile)
     const int32_t *pre_wtile;  // n+1 prefix of ceil(W/kWTile)
-    const int32_t *pre_itile;  // n+1 prefix of ceil(W/kTile) (first-window sort)
     const int32_t *pre_chunk;  // n+1 prefix of ceil(W/kChunk)
     unsigned long long *stats; // n * kNumStats per-stream counters, null when off
     int32_t *cell_pre;         // n+1 prefix of cells per stream (written by k_rows)
@@ -146,7 +145,7 @@ extern const char *const kPhaseNames[kNumPhases];
 hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t st, hipEvent_t *ev,
                         uint32_t phase_mask);
 // Enqueues the first-window load (sort of W points into the window arrays).
-hipError_t launch_init(const BatchArgs &a, int32_t itiles, int32_t passes, hipStream_t st);
+hipError_t launch_init(const BatchArgs &a, int32_t W, hipStream_t st);
 // One of a list of copies between pinned host memory and the device, of 4-byte
 // words; first: words of the copies before it.
 struct CopySeg {

@@ -386,10 +386,7 @@ static int stream_load(rtdbs_stream *s, const float *points, int64_t slides_done
     a.io1.in = s->d_in;
     a.io1.label = s->d_label;
     a.io1.cid = s->d_cid;
-    const int itiles = (int)((W + kTile - 1) / kTile);
-    int passes = ceil_log2(itiles);
-    if (passes % 2 == 0) passes++;  // result must land in the window arrays
-    HIPCHK(launch_init(a, itiles, passes, b->hs));
+    HIPCHK(launch_init(a, s->p.window, b->hs));
     HIPCHK(hipStreamSynchronize(b->hs));
     s->initialized = true;
     s->slides = slides_done;
@@ -495,7 +492,7 @@ static int batch_alloc(rtdbs_batch *b) {
     const int n = b->capacity;
     const size_t desc_b = ((size_t)n * sizeof(StreamDev) + 255) & ~size_t(255);
     const size_t io_b = ((size_t)n * sizeof(IO) + 255) & ~size_t(255);
-    const size_t pre_b = ((size_t)4 * (n + 1) * 4 + 255) & ~size_t(255);
+    const size_t pre_b = ((size_t)3 * (n + 1) * 4 + 255) & ~size_t(255);
     const size_t cnt_b = ((size_t)n * kNumStats * 8 + 255) & ~size_t(255);
     const size_t cpre_b = ((size_t)(n + 1) * 4 + 255) & ~size_t(255);
     HIPCHK(hipMalloc((void **)&b->dmem, desc_b + io_b + pre_b + cnt_b + 2 * cpre_b));
@@ -507,7 +504,7 @@ static int batch_alloc(rtdbs_batch *b) {
     b->d_stats = (unsigned long long *)(b->dmem + desc_b + io_b + pre_b);
     HIPCHK(hipHostMalloc((void **)&b->h_io, (size_t)n * sizeof(IO), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void **)&b->h_desc, (size_t)n * sizeof(StreamDev), hipHostMallocDefault));
-    HIPCHK(hipHostMalloc((void **)&b->h_pre, (size_t)4 * (n + 1) * 4, hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void **)&b->h_pre, (size_t)3 * (n + 1) * 4, hipHostMallocDefault));
     HIPCHK(hipStreamCreateWithFlags(&b->hs, hipStreamNonBlocking));
     return RTDBS_OK;
 }
@@ -610,7 +607,7 @@ int refresh_batch(rtdbs_batch *b) {
     if (b->hs) HIPCHK(hipStreamSynchronize(b->hs));
     StreamDev *desc = b->h_desc;
     int32_t *pre = b->h_pre;
-    std::memset(pre, 0, (size_t)4 * (n + 1) * 4);
+    std::memset(pre, 0, (size_t)3 * (n + 1) * 4);
     long long rows_total = 0, cells_total = 0;
     for (int i = 0; i < n; i++) {
         rtdbs_stream *s = b->streams[i];
@@ -618,11 +615,9 @@ int refresh_batch(rtdbs_batch *b) {
         const int st = (s->p.stride + kTile - 1) / kTile;
         const int wt = (s->p.window + kWTile - 1) / kWTile;
         const int ch = (s->p.window + kChunk - 1) / kChunk;
-        const int it = (s->p.window + kTile - 1) / kTile;
         pre[0 * (n + 1) + i + 1] = pre[0 * (n + 1) + i] + st;
         pre[1 * (n + 1) + i + 1] = pre[1 * (n + 1) + i] + wt;
         pre[2 * (n + 1) + i + 1] = pre[2 * (n + 1) + i] + ch;
-        pre[3 * (n + 1) + i + 1] = pre[3 * (n + 1) + i] + it;
         rows_total += (long long)s->p.window * s->R;
         cells_total += s->p.window;
         b->gens[i] = s->gen;
@@ -630,7 +625,7 @@ int refresh_batch(rtdbs_batch *b) {
     // asynchronous uploads from the pinned mirrors, ordered before the next
     // launch on the batch's stream
     HIPCHK(hipMemcpyAsync(b->d_desc, desc, (size_t)n * sizeof(StreamDev), hipMemcpyHostToDevice, b->hs));
-    HIPCHK(hipMemcpyAsync(b->d_pre, pre, (size_t)4 * (n + 1) * 4, hipMemcpyHostToDevice, b->hs));
+    HIPCHK(hipMemcpyAsync(b->d_pre, pre, (size_t)3 * (n + 1) * 4, hipMemcpyHostToDevice, b->hs));
     b->shape.stiles = pre[0 * (n + 1) + n];
     b->shape.wtiles = pre[1 * (n + 1) + n];
     b->shape.chunks = pre[2 * (n + 1) + n];
@@ -716,7 +711,6 @@ int refresh_batch(rtdbs_batch *b) {
     a.pre_stile = b->d_pre;
     a.pre_wtile = b->d_pre + (n + 1);
     a.pre_chunk = b->d_pre + 2 * (n + 1);
-    a.pre_itile = b->d_pre + 3 * (n + 1);
     a.stats = b->stats_on ? b->d_stats : nullptr;
     a.cell_pre = b->d_cell_pre;
     a.ctile_pre = b->d_ctile_pre;

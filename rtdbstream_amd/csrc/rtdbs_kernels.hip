@@ -345,30 +345,38 @@ __device__ __forceinline__ void sort_tile_keys(const KeyGrid &G, gptr<const floa
     bitonic_sort_regs<N, E>(v, lds, tid);
 }
 
-// First window: keys and coordinates of each sorted tile (init ping-pong A).
-__global__ __launch_bounds__(kTileThreads) void k_init_tiles(BatchArgs a) {
+// First window, launch 1: runs of kTile sorted keys, 16 waves per run (two keys
+// per thread), into the akey (sel 0) or skey (sel 1) half of the ping-pong.
+// A run is one serial chain of exchange stages, so a window of few runs takes
+// as long as one of them, however the rest of the device idles: with 4 waves
+// of 8 keys per thread this launch took 91 us at 200,000 points.
+constexpr int kInitThreads = kTile / 2;
+
+// Key of the first window's position p into the window arrays, with its
+// coordinates taken from the input: they are the same bytes as in the runs,
+// so the sort moves keys alone.
+__device__ __forceinline__ void init_place(const StreamDev &S, gptr<const float> in, int p, uint64_t key, int dim) {
+    const gptr<const float> c = in + (size_t)((uint32_t)key & slot_mask(S)) * dim;
+    gl(ldc(S.skey))[p] = key;
+    gl(ldc(S.sx))[p] = c[0];
+    if (dim > 1) gl(ldc(S.sy))[p] = c[1];
+    if (dim > 2) gl(ldc(S.sz))[p] = c[2];
+}
+
+template <bool LAST>
+__global__ __launch_bounds__(kInitThreads) void k_init_tiles(BatchArgs a, int sel) {
     __shared__ uint64_t lds[kTile];
-    const int g = blockIdx.x;
-    const int s = find_stream_c(a.pre_itile, a.n, g);
-    const StreamDev &S = a.s[s];
-    const IO io = a.use_io1 ? a.io1 : a.io[s];
-    const int tile0 = (g - ldc(a.pre_itile[s])) * kTile;
-    uint64_t v[8];
-    sort_tile_keys<kTile, 8>(key_grid(S), gl(io.in), ldc(S.W), tile0, 0, v, lds, threadIdx.x);
-    const int nvalid = min(kTile, S.W - tile0);
-    const uint32_t m = slot_mask(S);
-    const int dim = S.dim;
+    const StreamDev &S = a.s[0];
+    const int tile0 = blockIdx.x * kTile, W = ldc(S.W), dim = ldc(S.dim);
+    uint64_t v[2];
+    sort_tile_keys<kTile, 2>(key_grid(S), gl(a.io1.in), W, tile0, 0, v, lds, threadIdx.x);
+    const gptr<uint64_t> out = gl(sel ? ldc(S.skey) : ldc(S.akey));
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const int i = threadIdx.x * 8 + e;
-        if (i < nvalid) {
-            const int gi = (int)((uint32_t)v[e] & m);
-            const float *p = io.in + (size_t)gi * dim;
-            S.akey[tile0 + i] = v[e];
-            S.ax[tile0 + i] = p[0];
-            if (dim > 1) S.ay[tile0 + i] = p[1];
-            if (dim > 2) S.az[tile0 + i] = p[2];
-        }
+    for (int e = 0; e < 2; e++) {
+        const int i = tile0 + threadIdx.x * 2 + e;
+        if (i >= W) continue;
+        if (LAST) init_place(S, gl(a.io1.in), i, v[e], dim);
+        else out[i] = v[e];
     }
 }
 
@@ -641,9 +649,9 @@ struct MergeLds {
     uint64_t pred;
 };
 
-// Merges outputs [d0, d1) (d1 - d0 <= T) of merge(A, B) into m.out / m.src
-// (block-wide).
-template <int T>
+// Merges outputs [d0, d1) (d1 - d0 <= T) of merge(A, B) into m.out and, with
+// SRC, their sources into m.src (block-wide).
+template <int T, bool SRC = true>
 __device__ __forceinline__ void merge_tile(const uint64_t *A, int la, const uint64_t *B, int lb, int d0,
                                            int d1, MergeLds<T> &m, int *a0_out, int *b0_out) {
     const int tid = threadIdx.x;
@@ -681,11 +689,11 @@ __device__ __forceinline__ void merge_tile(const uint64_t *A, int la, const uint
             const bool takeA = (bi >= nb) || (ai < na && m.in[ai] < m.in[na + bi]);
             if (takeA) {
                 m.out[diag + q] = m.in[ai];
-                m.src[diag + q] = a0 + ai;
+                if (SRC) m.src[diag + q] = a0 + ai;
                 ai++;
             } else {
                 m.out[diag + q] = m.in[na + bi];
-                m.src[diag + q] = ~(b0 + bi);
+                if (SRC) m.src[diag + q] = ~(b0 + bi);
                 bi++;
             }
         }
@@ -695,34 +703,33 @@ __device__ __forceinline__ void merge_tile(const uint64_t *A, int la, const uint
     *b0_out = b0;
 }
 
-// One pass of the bottom-up merge sort of the first window: merges runs of
-// length L pairwise, ping-pong between akey (sel 0: a->s) and skey (sel 1).
+// One pass of the bottom-up merge sort of the first window's keys: merges runs
+// of length L pairwise, from akey (sel 0) or skey (sel 1) to the other; the
+// LAST pass ends in skey and places the coordinates. A pass of a window of
+// some 100,000 points is a chain of dependent loads (split searches, keys,
+// the merge in LDS), so the tiles are small enough to spread it over every
+// CU: 512 outputs per block.
+template <bool LAST>
 __global__ __launch_bounds__(kTileThreads) void k_init_merge(BatchArgs a, int L, int sel) {
-    __shared__ MergeLds<kTile> m;
-    const int g = blockIdx.x;
-    const int s = find_stream_c(a.pre_itile, a.n, g);
-    const StreamDev &S = a.s[s];
-    const int len = S.W;
-    const int o0 = (g - ldc(a.pre_itile[s])) * kTile;
-    const int o1 = min(o0 + kTile, len);
+    __shared__ MergeLds<kWTile> m;
+    const StreamDev &S = a.s[0];
+    const int len = ldc(S.W), dim = ldc(S.dim);
+    const int o0 = blockIdx.x * kWTile;
+    const int o1 = min(o0 + kWTile, len);
     const uint64_t *sk = sel == 0 ? S.akey : S.skey;
-    const float *sx = sel == 0 ? S.ax : S.sx, *sy = sel == 0 ? S.ay : S.sy, *sz = sel == 0 ? S.az : S.sz;
-    uint64_t *dk = sel == 0 ? S.skey : S.akey;
-    float *dx = sel == 0 ? S.sx : S.ax, *dy = sel == 0 ? S.sy : S.ay, *dz = sel == 0 ? S.sz : S.az;
+    const gptr<uint64_t> dk = gl(sel == 0 ? ldc(S.skey) : ldc(S.akey));
     const long long L2 = 2ll * L;
     const int base = (int)((o0 / L2) * L2);
     const int la = min(L, len - base);
     const int lb = min(L, len - base - la);
     int a0, b0;
-    merge_tile(sk + base, la, sk + base + la, lb, o0 - base, o1 - base, m, &a0, &b0);
-    const int dim = S.dim;
-    for (int i = threadIdx.x; i < o1 - o0; i += kTileThreads) {
-        const int sidx = m.src[i];
-        const int gi = sidx >= 0 ? base + sidx : base + la + ~sidx;
-        dk[o0 + i] = m.out[i];
-        dx[o0 + i] = sx[gi];
-        if (dim > 1) dy[o0 + i] = sy[gi];
-        if (dim > 2) dz[o0 + i] = sz[gi];
+    merge_tile<kWTile, false>(sk + base, la, sk + base + la, lb, o0 - base, o1 - base, m, &a0, &b0);
+#pragma unroll
+    for (int r = 0; r < kWTile / kTileThreads; r++) {
+        const int i = threadIdx.x + r * kTileThreads;
+        if (i >= o1 - o0) break;
+        if (LAST) init_place(S, gl(a.io1.in), o0 + i, m.out[i], dim);
+        else dk[o0 + i] = m.out[i];
     }
 }
 
@@ -2832,9 +2839,19 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
     return hipSuccess;
 }
 
-hipError_t launch_init(const BatchArgs &a, int32_t itiles, int32_t passes, hipStream_t st) {
-    RTDBS_LAUNCH(k_init_tiles, itiles, kTileThreads, a);
-    for (int p = 0; p < passes; p++) RTDBS_LAUNCH(k_init_merge, itiles, kTileThreads, a, kTile << p, p & 1);
+hipError_t launch_init(const BatchArgs &a, int32_t W, hipStream_t st) {
+    const int runs = (int)(((long long)W + kTile - 1) / kTile);
+    const int tiles = (int)(((long long)W + kWTile - 1) / kWTile);
+    int passes = 0;
+    while ((1ll << passes) < runs) passes++;
+    if (passes == 0) {
+        RTDBS_LAUNCH(k_init_tiles<true>, runs, kInitThreads, a, 1);
+        return hipSuccess;
+    }
+    RTDBS_LAUNCH(k_init_tiles<false>, runs, kInitThreads, a, (passes - 1) & 1);
+    for (int p = 0; p + 1 < passes; p++)
+        RTDBS_LAUNCH(k_init_merge<false>, tiles, kTileThreads, a, kTile << p, (passes - 1 - p) & 1);
+    RTDBS_LAUNCH(k_init_merge<true>, tiles, kTileThreads, a, kTile << (passes - 1), 0);
     return hipSuccess;
 }
 
