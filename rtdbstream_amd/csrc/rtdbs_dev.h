@@ -145,7 +145,20 @@ extern const char *const kPhaseNames[kNumPhases];
 hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t st, hipEvent_t *ev,
                         uint32_t phase_mask);
 // Enqueues the first-window load (sort of W points into the window arrays).
-hipError_t launch_init(const BatchArgs &a, int32_t W, hipStream_t st);
+
+// Pinned host memory that kernels write: the bounds of a first window per
+// block (low then high per axis), and the window-read's check.
+constexpr int kBoundBlocks = 128;
+struct FirstWindow {
+    float bnd[kBoundBlocks * 6];
+    int32_t bad;
+};
+hipError_t launch_bounds_of(const float *in, int32_t W, int32_t dim, float *bnd, hipStream_t st);
+// t, u: slides completed and ring unit the stream starts with
+hipError_t launch_init(const BatchArgs &a, int32_t W, int32_t t, int32_t u, hipStream_t st);
+// Window of the only stream in slot order, W x dim floats; *bad set to 1 where
+// a position's slot is outside the window.
+hipError_t launch_window_out(const BatchArgs &a, int32_t W, float *out, int32_t *bad, hipStream_t st);
 // One of a list of copies between pinned host memory and the device, of 4-byte
 // words; first: words of the copies before it.
 struct CopySeg {

@@ -287,7 +287,15 @@ namespace rtdbs {
 // key bits run out. Only beyond that are the axes shrunk, proportionally, and
 // points outside clamped into the border cells, which keeps the search exact
 // (never dense or safe) but slower.
-static void set_geometry(rtdbs_stream *s, const float *pts) {
+static bool bounds_given(const rtdbs_params &p) {
+    for (int a = 0; a < p.dim; a++)
+        if (!(p.hi[a] > p.lo[a])) return false;
+    return true;
+}
+
+// bnd: kBoundBlocks partial bounds of the first window (launch_bounds_of), or
+// nullptr where the parameters give the bounds
+static void set_geometry(rtdbs_stream *s, const float *bnd) {
     const rtdbs_params &p = s->p;
     const int d = p.dim;
     s->side = (double)p.eps / (double)s->k * (1.0 + 1.0 / 65536.0);
@@ -295,9 +303,7 @@ static void set_geometry(rtdbs_stream *s, const float *pts) {
     const int key_bits = std::min(52, 64 - s->slot_bits);
     const double key_cells = std::ldexp(1.0, key_bits);
     const double axis_cap = std::ldexp(1.0, 30);
-    bool given = true;
-    for (int a = 0; a < d; a++)
-        if (!(p.hi[a] > p.lo[a])) given = false;
+    const bool given = bounds_given(p);
     double mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
     for (int a = 0; a < d; a++) {
         if (given) {
@@ -305,10 +311,9 @@ static void set_geometry(rtdbs_stream *s, const float *pts) {
             mx[a] = p.hi[a];
         } else {
             float lo = INFINITY, hi = -INFINITY;
-            for (int i = 0; i < p.window; i++) {
-                const float v = pts[(size_t)i * d + a];
-                if (v < lo) lo = v;
-                if (v > hi) hi = v;
+            for (int i = 0; i < kBoundBlocks; i++) {
+                lo = std::min(lo, bnd[i * 6 + a]);
+                hi = std::max(hi, bnd[i * 6 + 3 + a]);
             }
             if (!(hi >= lo)) lo = hi = 0.0f;  // all NaN
             mn[a] = lo;
@@ -360,6 +365,10 @@ static void set_geometry(rtdbs_stream *s, const float *pts) {
 
 }  // namespace rtdbs
 
+namespace rtdbs {
+static int new_solo(rtdbs_stream *s);
+}
+
 static int stream_load(rtdbs_stream *s, const float *points, int64_t slides_done) {
     if (!s) return fail(RTDBS_EINVAL, "stream is NULL");
     if (!points) return fail(RTDBS_EINVAL, "points is NULL");
@@ -369,24 +378,27 @@ static int stream_load(rtdbs_stream *s, const float *points, int64_t slides_done
         int rc = batch_sync(s->solo);
         if (rc) return rc;
     }
-    set_geometry(s, points);
-    s->gen = next_generation();
-    int rc = ensure_solo(s);
+    int rc = new_solo(s);
     if (rc) return rc;
     rtdbs_batch *b = s->solo;
-    rc = refresh_batch(b);
-    if (rc) return rc;
     const size_t W = (size_t)s->p.window, d = (size_t)s->p.dim;
     const int units = s->p.window / s->p.stride;
     HIPCHK(hipMemcpyAsync(s->d_in, points, W * d * 4, hipMemcpyHostToDevice, b->hs));
-    StreamMut m0 = {(int32_t)(slides_done % (1 << 30)), (int32_t)(slides_done % units), 0, {0, 0, 0, 0, 0}};
-    HIPCHK(hipMemcpyAsync(s->dev.mut, &m0, sizeof(m0), hipMemcpyHostToDevice, b->hs));
+    const bool given = bounds_given(s->p);
+    if (!given) {
+        HIPCHK(launch_bounds_of(s->d_in, s->p.window, s->p.dim, b->h_first->bnd, b->hs));
+        HIPCHK(hipStreamSynchronize(b->hs));
+    }
+    set_geometry(s, given ? nullptr : b->h_first->bnd);
+    s->gen = next_generation();
+    rc = batch_set_members(b, &s, 1);
+    if (rc) return rc;
     BatchArgs a = b->args;
     a.use_io1 = 1;
     a.io1.in = s->d_in;
     a.io1.label = s->d_label;
     a.io1.cid = s->d_cid;
-    HIPCHK(launch_init(a, s->p.window, b->hs));
+    HIPCHK(launch_init(a, s->p.window, (int32_t)(slides_done % (1 << 30)), (int32_t)(slides_done % units), b->hs));
     HIPCHK(hipStreamSynchronize(b->hs));
     s->initialized = true;
     s->slides = slides_done;
@@ -453,22 +465,13 @@ extern "C" int rtdbs_stream_get_window(rtdbs_stream *s, float *points) {
         int rc = batch_sync(s->solo);
         if (rc) return rc;
     }
-    const size_t W = (size_t)s->p.window;
-    const int d = s->p.dim;
-    std::vector<uint64_t> key(W);
-    std::vector<float> c[3];
-    HIPCHK(hipMemcpy(key.data(), s->dev.skey, W * 8, hipMemcpyDeviceToHost));
-    const float *src[3] = {s->dev.sx, s->dev.sy, s->dev.sz};
-    for (int a = 0; a < d; a++) {
-        c[a].resize(W);
-        HIPCHK(hipMemcpy(c[a].data(), src[a], W * 4, hipMemcpyDeviceToHost));
-    }
-    const uint64_t m = (1ull << s->slot_bits) - 1ull;
-    for (size_t i = 0; i < W; i++) {
-        const size_t slot = (size_t)(key[i] & m);
-        if (slot >= W) return fail(RTDBS_EHIP, "corrupt window state");
-        for (int a = 0; a < d; a++) points[slot * d + a] = c[a][i];
-    }
+    // d_in is the upload area of host-buffer calls, which have returned
+    rtdbs_batch *b = s->solo;
+    b->h_first->bad = 0;
+    HIPCHK(launch_window_out(b->args, s->p.window, s->d_in, &b->h_first->bad, b->hs));
+    HIPCHK(hipStreamSynchronize(b->hs));
+    if (b->h_first->bad) return fail(RTDBS_EHIP, "corrupt window state");
+    HIPCHK(hipMemcpy(points, s->d_in, (size_t)s->p.window * s->p.dim * 4, hipMemcpyDeviceToHost));
     return RTDBS_OK;
 }
 
@@ -502,9 +505,11 @@ static int batch_alloc(rtdbs_batch *b) {
     b->d_io = (IO *)(b->dmem + desc_b);
     b->d_pre = (int32_t *)(b->dmem + desc_b + io_b);
     b->d_stats = (unsigned long long *)(b->dmem + desc_b + io_b + pre_b);
-    HIPCHK(hipHostMalloc((void **)&b->h_io, (size_t)n * sizeof(IO), hipHostMallocDefault));
-    HIPCHK(hipHostMalloc((void **)&b->h_desc, (size_t)n * sizeof(StreamDev), hipHostMallocDefault));
-    HIPCHK(hipHostMalloc((void **)&b->h_pre, (size_t)3 * (n + 1) * 4, hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void **)&b->hmem, desc_b + io_b + pre_b + sizeof(FirstWindow), hipHostMallocDefault));
+    b->h_desc = (StreamDev *)b->hmem;
+    b->h_io = (IO *)(b->hmem + desc_b);
+    b->h_pre = (int32_t *)(b->hmem + desc_b + io_b);
+    b->h_first = (FirstWindow *)(b->hmem + desc_b + io_b + pre_b);
     HIPCHK(hipStreamCreateWithFlags(&b->hs, hipStreamNonBlocking));
     return RTDBS_OK;
 }
@@ -571,9 +576,7 @@ void batch_free(rtdbs_batch *b) {
     for (hipEvent_t e : b->ev_ring)
         if (e) (void)hipEventDestroy(e);
     if (b->hs) (void)hipStreamDestroy(b->hs);
-    if (b->h_io) (void)hipHostFree(b->h_io);
-    if (b->h_desc) (void)hipHostFree(b->h_desc);
-    if (b->h_pre) (void)hipHostFree(b->h_pre);
+    if (b->hmem) (void)hipHostFree(b->hmem);
     if (b->h_stage) (void)hipHostFree(b->h_stage);
     if (b->h_segs) (void)hipHostFree(b->h_segs);
     if (b->d_xfer) (void)hipFree(b->d_xfer);
@@ -741,20 +744,20 @@ static int batch_check_current(rtdbs_batch *b) {
     return RTDBS_OK;
 }
 
-int ensure_solo(rtdbs_stream *s) {
+static int new_solo(rtdbs_stream *s) {
     if (s->solo) return RTDBS_OK;
     int rc = 0;
     rtdbs_batch *b = batch_new(1, false, &rc);
     if (!b) return rc;
     b->solo = true;
-    rtdbs_stream *one[1] = {s};
-    rc = batch_set_members(b, one, 1);
-    if (rc) {
-        batch_free(b);
-        return rc;
-    }
     s->solo = b;
     return RTDBS_OK;
+}
+
+int ensure_solo(rtdbs_stream *s) {
+    if (s->solo && s->solo->n) return RTDBS_OK;
+    const int rc = new_solo(s);
+    return rc ? rc : batch_set_members(s->solo, &s, 1);
 }
 
 // Event set for the next timed slide (reads the full ring first).

@@ -54,6 +54,8 @@ struct rtdbs_batch {
     bool io_valid = false;
     rtdbs::StreamDev *h_desc = nullptr;  // pinned mirrors of the descriptor and prefix tables
     int32_t *h_pre = nullptr;            // (uploaded asynchronously on the batch's stream)
+    rtdbs::FirstWindow *h_first = nullptr;  // pinned results of the first-window and window-read kernels
+    char *hmem = nullptr;                // the pinned allocation they share
     // Host-buffer slides. The device side of each member's I/O (stage_io): the
     // stream's own arena buffers in a solo batch, else one contiguous transfer
     // area holding every member's stride (in_off), then its label and cid

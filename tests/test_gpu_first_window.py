@@ -27,3 +27,33 @@ def test_sizes(engine, oracle, dim, W, S):
             l, c = s.slide(data[W + t * S: W + (t + 1) * S])
             assert np.array_equal(l, rl[t]) and np.array_equal(c, rc[t]), (again, t)
     s.close()
+
+
+# bounds of the first window, as the grid's origin shows them: extremes in the
+# first, last and every other place of the scan (32,768 points a turn), NaNs
+# passed over, an axis of NaNs alone taken as zero
+@pytest.mark.parametrize("W", [1, 2, 63, 257, 32768, 32769, 70001])
+@pytest.mark.parametrize("dim", [1, 2, 3])
+@pytest.mark.parametrize("nans", ["none", "some", "axis"])
+def test_bounds(engine, dim, W, nans):
+    rng = np.random.default_rng(W)
+    eps = 0.5
+    for place in sorted({0, W // 2, W - 1}):
+        x = rng.uniform(-1, 1, (W, dim)).astype(np.float32)
+        x[place] = -3.25
+        x[W - 1 - place] = 7.5
+        if nans == "some":
+            x[rng.integers(0, W, W // 3)] = np.nan
+        elif nans == "axis":
+            x[:, dim - 1] = np.nan
+        s = engine.Stream(dim, W, W, eps, 3)
+        s.init(x)
+        info = s.info()
+        for a in range(dim):
+            v = x[:, a][~np.isnan(x[:, a])].astype(np.float64)
+            mn, mx = (v.min(), v.max()) if v.size else (0.0, 0.0)
+            lo = float(np.float32(mn - 2.0 * (mx - mn) - eps))
+            assert info["lo"][a] == lo, (place, a)
+            assert info["grid"][a] == int((mx + 2.0 * (mx - mn) + eps - lo) * (1.0 / info["cell_side"])) + 1, (place, a)
+        assert np.array_equal(s.window().reshape(W, dim).view(np.uint32), x.view(np.uint32))
+        s.close()
