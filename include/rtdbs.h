@@ -338,7 +338,7 @@ typedef struct {
     int64_t merge_pairs;   /* touching element pairs found by the merge */
     int32_t cell_parallel; /* 1: count and border ran cell-parallel; 0: either ran point-parallel (large
                               batches). The merge counters come from the cell-parallel merge,
-                              which both paths use by default */
+                              which both paths use */
     int32_t pad;
     int64_t reserved[6];
 } rtdbs_stats;
@@ -353,7 +353,9 @@ int rtdbs_stream_set_stats(rtdbs_stream *s, int enable);
 int rtdbs_stream_get_stats(rtdbs_stream *s, rtdbs_stats *out);
 
 /* Event timing on a batch (or a stream's solo batch): enable = 0 off,
- * 1 every phase, 2 only the range-count kernel (two events per slide). */
+ * 1 every phase, 2 only the range-count kernel (two events per slide). With 1,
+ * streams of up to 4096 points are updated by the separate kernels of the
+ * larger ones, whose phases are timed, instead of by one kernel. */
 int rtdbs_batch_set_timing(rtdbs_batch *b, int enable);
 int rtdbs_stream_set_timing(rtdbs_stream *s, int enable);
 /* Accumulated milliseconds and launch counts per phase since the last reset.

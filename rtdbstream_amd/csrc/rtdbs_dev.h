@@ -15,6 +15,11 @@ constexpr int kTile = 2048;        // positions per sort tile (stride, first win
 constexpr int kWTile = 512;        // positions per window tile: expiry, merge, cell table
 constexpr int kTileThreads = 256;  // threads per tile block
 constexpr int kChunk = 64;         // positions per wave in the neighbourhood kernels
+// streams whose update one block does in LDS (k_update_small)
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallPer = 4;                           // most window positions per thread
+constexpr int kSmallW = kSmallPer * kSmallThreads;     // largest window
+constexpr int kSmallS = kSmallThreads;                 // largest stride
 constexpr int kCap = 512;          // candidates staged in LDS per wave
 constexpr int kMaxK = 3;           // largest stencil reach
 constexpr int kMaxRows = 49;       // (2k+1)^(dim-1) for k <= 3, dim <= 3
@@ -123,6 +128,7 @@ struct LaunchShape {
     int32_t link;            // 1: some stream has safe cells: merged by k_merge_cells
     int32_t unsafe;          // 1: some stream has none (reach 1): merged by k_union
     int32_t link_blocks;     // blocks of k_merge_cells and k_cell_cores
+    int32_t small_update;    // window positions per thread of the one-block update in LDS (k_update_small), 0: not used
     int32_t rank_split;      // 1: stride rank with 64-key blocks (small strides), 0: 256-key blocks
     int32_t border_regroup;  // point-parallel outputs: 1 one lane per core, non-cores regrouped onto 4 lanes
 };

@@ -612,9 +612,13 @@ int refresh_batch(rtdbs_batch *b) {
     int32_t *pre = b->h_pre;
     std::memset(pre, 0, (size_t)3 * (n + 1) * 4);
     long long rows_total = 0, cells_total = 0;
+    bool small = true;  // every stream fits the one-block update
+    int most = 0;       // points of the largest window
     for (int i = 0; i < n; i++) {
         rtdbs_stream *s = b->streams[i];
         desc[i] = s->dev;
+        most = std::max(most, (int)s->p.window);
+        small = small && s->p.window <= kSmallW && s->p.stride <= kSmallS;
         const int st = (s->p.stride + kTile - 1) / kTile;
         const int wt = (s->p.window + kWTile - 1) / kWTile;
         const int ch = (s->p.window + kChunk - 1) / kChunk;
@@ -632,6 +636,10 @@ int refresh_batch(rtdbs_batch *b) {
     b->shape.stiles = pre[0 * (n + 1) + n];
     b->shape.wtiles = pre[1 * (n + 1) + n];
     b->shape.chunks = pre[2 * (n + 1) + n];
+    // window update: one block per stream where all of them fit one
+    // (RTDBS_SMALL_UPDATE: 0 forces the separate kernels)
+    b->shape.small_update =
+        small && env_int("RTDBS_SMALL_UPDATE", 1, 0, 1) ? (most + kSmallThreads - 1) / kSmallThreads : 0;
     // stride rank: 64-key blocks when 256-key blocks would not cover the device
     // (RTDBS_RANK_SPLIT: 0 forces 256-key blocks, 1 the 64-key form)
     const int rsplit = env_int("RTDBS_RANK_SPLIT", -1, 0, 1);

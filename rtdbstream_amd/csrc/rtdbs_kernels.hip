@@ -248,6 +248,12 @@ __device__ __forceinline__ void divmod_key(uint64_t x, int64_t d, int64_t *q, in
 // sorting: register bitonic tile sort, rank merge of the stride's tiles,
 // merge-path merges of the window
 
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, l);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), l);
+    return ((uint64_t)hi << 32) | lo;
+}
+
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
     const int lo = xor_lane((int)(uint32_t)v, m);
     const int hi = xor_lane((int)(uint32_t)(v >> 32), m);
@@ -904,6 +910,221 @@ __global__ __launch_bounds__(kTileThreads) void k_cells(BatchArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// window update of small streams: one block per stream, the window's keys in LDS
+
+// Inclusive prefix sum over a wave's lanes, in registers (all lanes active).
+__device__ __forceinline__ int wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast 15, 31
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+
+// Flags of a block in position order (round r, wave, lane), counted per round
+// and wave in cnt[r * 16 + wave]: before[r] = the flags before this wave's of
+// round r; returns the total. Every wave scans the PER * 16 <= 128 counts, two
+// per lane, for itself. Starts with the barrier that the counts need.
+template <int PER>
+__device__ __forceinline__ int small_scan(const int *cnt, int wv, int (&before)[PER]) {
+    __syncthreads();
+    const int lane = lane_id();
+    const int c0 = 2 * lane < PER * 16 ? cnt[2 * lane] : 0, c1 = 2 * lane < PER * 16 ? cnt[2 * lane + 1] : 0;
+    const int x = wave_scan(c0 + c1);
+    const int e = (wv & 1) ? x - c1 : x - c0 - c1;
+#pragma unroll
+    for (int r = 0; r < PER; r++) before[r] = __builtin_amdgcn_readlane(e, r * 8 + (wv >> 1));
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Number of the len <= 4 * q sorted keys a[0, len) in LDS below key (q a power
+// of four; last: the last index of a that may be read). Three probes a step:
+// a step is one LDS latency, and the latency is what it costs.
+__device__ __forceinline__ int small_below(const uint64_t *a, int len, int last, int q, uint64_t key) {
+    auto below = [&](int i) { return ((i < len) & (a[min(i, last)] < key)) ? 1 : 0; };
+    int n = q * (below(q - 1) + below(2 * q - 1) + below(3 * q - 1) + below(4 * q - 1));
+    for (q >>= 2; q > 0; q >>= 2) n += q * (below(n + q - 1) + below(n + 2 * q - 1) + below(n + 3 * q - 1));
+    return n;
+}
+
+// The whole update of a stream of up to PER * 1024 points and kSmallS points a
+// stride: what k_sort_expire, k_rank, k_merge_final and k_cells do together.
+// At these sizes each of those is a launch and a chain of a few dependent
+// round trips through memory; here the chain is the window's keys and the
+// stride in, then LDS, then the new window out. A whole slide of 1,000 points
+// and strides of 10 in 2-D, resident on the device: 42 us with the separate
+// kernels, 32 us so; 4,000 and 400: 46.5 and 41.5 us, 64 such streams of 2,000:
+// 71 and 60 us. Past 4,096 points one block's share of the work is the longer
+// (8,000 and 800: 48 and 51 us with eight positions per thread). A survivor's
+// place is its
+// rank among the survivors plus the stride keys below it, a stride key's its
+// rank in the sorted stride plus the survivors below it.
+template <int PER>
+__global__ __launch_bounds__(kSmallThreads) void k_update_small(BatchArgs a) {
+    __shared__ uint64_t sk[PER * kSmallThreads];  // survivors' keys, then the window's
+    __shared__ uint64_t bk[kSmallS + 8];          // the stride's keys, sorted, then ~0
+    __shared__ float bc[3][kSmallS];              // its coordinates, as they came
+    __shared__ int cnt[2][PER * 16];
+    static_assert(kSmallS == kSmallThreads && kSmallThreads == 1024 && PER <= 4, "");
+    const int s = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wv = uni(tid >> 6);
+    const StreamDev &S = a.s[s];
+    const int W = ldc(S.W), SS = ldc(S.S), dim = ldc(S.dim), sb = ldc(S.slot_bits);
+    const gptr<uint64_t> skey = gl(ldc(S.skey));
+    const gptr<float> sx = gl(ldc(S.sx)), sy = gl(ldc(S.sy)), sz = gl(ldc(S.sz));
+    const uint32_t sm = (uint32_t)((1ull << sb) - 1ull);
+    const int lo_slot = ldc(ldc(S.mut)->u) * SS;
+    const uint64_t lower = (1ull << lane) - 1ull;
+    const IO io = a.use_io1 ? a.io1 : a.io[s];
+    // the stride and the window, every load issued before the sort
+    const gptr<const float> in = gl(io.in) + (size_t)min(tid, SS - 1) * dim;
+    const float n0 = in[0], n1 = dim > 1 ? in[1] : 0.f, n2 = dim > 2 ? in[2] : 0.f;
+    uint64_t key[PER];
+    float cx[PER], cy[PER], cz[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int p = min(r * kSmallThreads + tid, W - 1);
+        key[r] = skey[p];
+        cx[r] = sx[p];
+        cy[r] = dim > 1 ? sy[p] : 0.f;
+        cz[r] = dim > 2 ? sz[p] : 0.f;
+    }
+    bc[0][tid] = n0;
+    bc[1][tid] = n1;
+    bc[2][tid] = n2;
+    uint64_t v[1] = {tid < SS ? (cell_key_g(key_grid(S), n0, n1, n2) << sb) | (uint64_t)(lo_slot + tid) : ~0ull};
+    // the stride sorted: runs of 64 in each wave's lanes, then merged pairwise,
+    // each key moving to its place in its run plus the partner run's keys below
+    // it; the padding keys stay last
+    if (wv * 64 < SS) bitonic_sort_regs<64, 1>(v, nullptr, lane);
+    bk[tid] = v[0];
+    if (tid < 8) bk[kSmallS + tid] = ~0ull;
+    for (int L = 64, q = 16; L < SS; L <<= 1) {
+        __syncthreads();
+        v[0] = bk[tid];
+        const int run = tid & ~(L - 1), other = run ^ L;
+        int to = (run & other) + (tid - run);
+        if (wv * 64 < SS) to += small_below(bk + other, min(max(SS - other, 0), L), kSmallS - 1 - other, q, v[0]);
+        __syncthreads();
+        if (tid < SS) bk[to] = v[0];
+        if (4 * q < 2 * L) q <<= 2;
+    }
+    // survivors in order
+    int at[PER], before[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int slot = (int)((uint32_t)key[r] & sm);
+        const bool f = r * kSmallThreads + tid < W && (slot < lo_slot || slot >= lo_slot + SS);
+        const uint64_t m = __ballot(f);
+        at[r] = f ? __popcll(m & lower) : -1;
+        if (lane == 0) cnt[0][r * 16 + wv] = __popcll(m);
+    }
+    small_scan<PER>(cnt[0], wv, before);  // from its barrier on bk is whole
+    v[0] = bk[tid];
+    const int ns = W - SS;
+#pragma unroll
+    for (int r = 0; r < PER; r++)
+        if (at[r] >= 0) {
+            at[r] += before[r];
+            sk[at[r]] = key[r];
+        }
+    // Survivors' places. A wave's 64 window keys rise with the lane, so the
+    // stride keys between the first and the last bound every lane's count; few
+    // of them as a rule, compared one by one.
+    const uint64_t sample = bk[lane * 16 + 15];
+    uint64_t near[PER];
+    int nb[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const uint64_t k0 = readlane64(key[r], 0), k1 = readlane64(key[r], 63);
+        const int b0 = 16 * __popcll(__ballot(sample < k0)), b1 = 16 * __popcll(__ballot(sample < k1));
+        nb[r] = lane < 32 ? b0 : b1;
+        near[r] = bk[min(nb[r] + (lane & 15), kSmallS - 1)];
+    }
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const uint64_t k0 = readlane64(key[r], 0), k1 = readlane64(key[r], 63);
+        const uint64_t bel = __ballot(near[r] < (lane < 32 ? k0 : k1));
+        // past the array's end (every key below) the last key repeats
+        const int lo = min(__builtin_amdgcn_readlane(nb[r], 0) + __popcll(bel & 0xffffull), kSmallS);
+        const int hi = min(__builtin_amdgcn_readlane(nb[r], 63) + __popcll(bel & 0xffff00000000ull), kSmallS);
+        int n = lo;
+        if (hi - lo <= 8) {  // keys past hi are above every lane's
+            uint64_t t[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) t[j] = bk[lo + j];
+#pragma unroll
+            for (int j = 0; j < 8; j++) n += t[j] < key[r] ? 1 : 0;
+        } else {
+            n += small_below(bk + lo, hi - lo, hi - lo, hi - lo <= 64 ? 16 : 256, key[r]);
+        }
+        if (at[r] >= 0) at[r] += n;
+    }
+    __syncthreads();  // sk holds the survivors
+    int bat = -1;
+    if (wv * 64 < SS) {
+        bat = tid + small_below(sk, ns, PER * kSmallThreads - 1, PER == 1 ? 256 : 1024, v[0]);
+        if (tid >= SS) bat = -1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; r++)
+        if (at[r] >= 0) {
+            sk[at[r]] = key[r];
+            skey[at[r]] = key[r];
+            sx[at[r]] = cx[r];
+            if (dim > 1) sy[at[r]] = cy[r];
+            if (dim > 2) sz[at[r]] = cz[r];
+        }
+    if (bat >= 0) {
+        const int j = (int)((uint32_t)v[0] & sm) - lo_slot;
+        sk[bat] = v[0];
+        skey[bat] = v[0];
+        sx[bat] = bc[0][j];
+        if (dim > 1) sy[bat] = bc[1][j];
+        if (dim > 2) sz[bat] = bc[2][j];
+    }
+    __syncthreads();
+    // cell table
+    uint64_t prev[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int p = r * kSmallThreads + tid;
+        key[r] = sk[min(p, W - 1)];
+        prev[r] = sk[max(min(p, W) - 1, 0)];
+    }
+    uint32_t starts = 0;  // bit r: position r * 1024 + tid starts a cell
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int p = r * kSmallThreads + tid;
+        const bool f = p < W && (p == 0 || (key[r] >> sb) != (prev[r] >> sb));
+        const uint64_t m = __ballot(f);
+        at[r] = __popcll(m & lower) + (f ? 1 : 0) - 1;
+        starts |= (uint32_t)f << r;
+        if (lane == 0) cnt[1][r * 16 + wv] = __popcll(m);
+    }
+    const int ncell = small_scan<PER>(cnt[1], wv, before);
+    const gptr<int32_t> pcell = gl(ldc(S.pcell)), cstart = gl(ldc(S.cstart));
+    const gptr<uint64_t> ckey = gl(ldc(S.ckey));
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int p = r * kSmallThreads + tid;
+        if (p >= W) continue;
+        const int c = at[r] + before[r];
+        pcell[p] = c;
+        if ((starts >> r) & 1u) {
+            cstart[c] = p;
+            ckey[c] = key[r] >> sb;
+        }
+    }
+    if (tid == 0) {
+        ldc(S.mut)->ncell = ncell;
+        cstart[ncell] = W;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // stencil rows: for every cell and every row of its (2k+1)^dim stencil, the
 // contiguous range of window positions holding that row's cells. A row varies
 // the last used axis, whose key stride is 1 (unused axes have extent 1 and
@@ -946,12 +1167,6 @@ __device__ __forceinline__ RowsView rows_view(const StreamDev &S) {
     v.dense_ok = ldc(S.dense_ok);
     v.ncell = ldc(ldc(S.mut)->ncell);  // written by the cell-table kernel
     return v;
-}
-
-__device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, l);
-    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), l);
-    return ((uint64_t)hi << 32) | lo;
 }
 
 // Ranks (number of keys below) of two wave-uniform keys in the sorted
@@ -2840,6 +3055,14 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
     hipError_t e;
 #define PH_BEGIN(ph) if ((e = mark(ev, phase_mask, 2 * (ph), st)) != hipSuccess) return e
 #define PH_END(ph) if ((e = mark(ev, phase_mask, 2 * (ph) + 1, st)) != hipSuccess) return e
+    // per-phase times of the window update are of its separate kernels
+    constexpr uint32_t kUpdatePhases =
+        (1u << kPhStrideSort) | (1u << kPhMerge) | (1u << kPhMergeFinal) | (1u << kPhCells);
+    if (sh.small_update && !(ev && (phase_mask & kUpdatePhases))) {
+        if (sh.small_update == 1) RTDBS_LAUNCH(k_update_small<1>, a.n, kSmallThreads, a);
+        else if (sh.small_update == 2) RTDBS_LAUNCH(k_update_small<2>, a.n, kSmallThreads, a);
+        else RTDBS_LAUNCH(k_update_small<kSmallPer>, a.n, kSmallThreads, a);
+    } else {
     PH_BEGIN(kPhStrideSort);
     RTDBS_LAUNCH(k_sort_expire, sh.stiles * kSortParts + sh.wtiles, kTileThreads, a);
     PH_END(kPhStrideSort);
@@ -2858,6 +3081,7 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
     PH_BEGIN(kPhCells);
     RTDBS_LAUNCH(k_cells, sh.wtiles, kTileThreads, a);
     PH_END(kPhCells);
+    }
     PH_BEGIN(kPhRows);
     RTDBS_LAUNCH(k_rows, sh.rows_blocks + 1, kTileThreads, a);
     PH_END(kPhRows);
