@@ -61,3 +61,26 @@ def test_batches(engine, oracle, sizes, graph):
     b.close()
     for s in st:
         s.close()
+
+
+# host slides of a small stream read and write pinned memory from the kernels:
+# the caller's buffers where they are pinned, else the engine's staging
+@pytest.mark.parametrize("pinned", [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)])
+@pytest.mark.parametrize("shift", [0, 2])  # bytes off a word
+def test_host_buffers(engine, oracle, pinned, shift):
+    W, S, slides, eps, mp = 1500, 300, 6, 0.25, 4
+    d = _data(2, W, S, slides)
+    rl, rc = oracle.stream(d, W, S, eps, mp, slides, method="bruteforce")
+    s = engine.Stream(2, W, S, eps, mp, lo=[-50.0] * 2, hi=[50.0] * 2)
+    s.init(d[:W])
+    hb = engine.HostBuffer(S * 8 + W * 8 + shift)
+    x = hb.array(np.float32, S * 2, offset=shift) if pinned[0] else np.empty(S * 2, np.float32)
+    l = hb.array(np.int32, W, offset=S * 8 + shift) if pinned[1] else np.empty(W, np.int32)
+    c = hb.array(np.int32, W, offset=S * 8 + W * 4 + shift) if pinned[2] else np.empty(W, np.int32)
+    for t in range(slides):
+        x[:] = d[W + t * S: W + (t + 1) * S].reshape(-1)
+        l[:] = -7
+        c[:] = -7
+        s.slide(x, l, c)
+        assert np.array_equal(l, rl[t]) and np.array_equal(c, rc[t]), t
+    s.close()
