@@ -45,6 +45,7 @@ constexpr uint8_t kFlagDense = 2;
 constexpr uint8_t kCellSafe = 1;
 constexpr uint8_t kCellDense = 2;
 constexpr int kNoCore = 0x7fffffff;  // fcore of a cell without cores
+
 // Per-stream state that the device itself advances every slide.
 struct StreamMut {
     int32_t t;       // slides completed
@@ -77,6 +78,7 @@ struct StreamDev {
     float *ax, *ay, *az;
     // stride: sorted tiles (keys, bkey0), then the sorted stride (B1)
     uint64_t *bkey0;
+    uint64_t *bends;  // first and last key of each 64 of bkey0
     uint64_t *bkey1;
     float *bx1, *by1, *bz1;
     // cell table

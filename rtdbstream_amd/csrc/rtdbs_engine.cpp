@@ -113,7 +113,7 @@ int validate_params(const rtdbs_params *p) {
 // Buffer layout of one stream's device arena.
 struct Layout {
     size_t off_mut, off_skey, off_sx, off_sy, off_sz, off_akey, off_ax, off_ay, off_az;
-    size_t off_bkey0, off_bkey1, off_bx1, off_by1, off_bz1;
+    size_t off_bkey0, off_bends, off_bkey1, off_bx1, off_by1, off_bz1;
     size_t off_cstart, off_ckey, off_pcell, off_rows, off_cflag, off_fcore, off_flags, off_uf,
         off_tile_a, off_tile_b, off_in, off_label, off_cid;
     size_t total;
@@ -143,6 +143,7 @@ static Layout make_layout(const rtdbs_params &p, int R) {
     L.off_ay = d > 1 ? take(wc) : 0;
     L.off_az = d > 2 ? take(wc) : 0;
     L.off_bkey0 = take(S * 8);
+    L.off_bends = take((S + 511) / 512 * 8 * 16);
     L.off_bkey1 = take(S * 8);
     L.off_bx1 = take(S * 4);
     L.off_by1 = d > 1 ? take(S * 4) : 0;
@@ -251,6 +252,7 @@ extern "C" int rtdbs_stream_create(const rtdbs_params *params, rtdbs_stream **ou
     D.ay = f(L.off_ay, d > 1);
     D.az = f(L.off_az, d > 2);
     D.bkey0 = (uint64_t *)(A + L.off_bkey0);
+    D.bends = (uint64_t *)(A + L.off_bends);
     D.bkey1 = (uint64_t *)(A + L.off_bkey1);
     D.bx1 = f(L.off_bx1, true);
     D.by1 = f(L.off_by1, d > 1);

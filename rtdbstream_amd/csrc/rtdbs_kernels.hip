@@ -475,15 +475,25 @@ __device__ __forceinline__ void expire_count(const BatchArgs &a, int g, int *lds
 
 // Launch 1 of a slide: the first kSortParts blocks of each stride tile sort
 // the stride by key (the reference's compute_cell_id + sortByCellIdAndOrder,
-// aabb.cu:589-611, thrust_helper.cu:21-29) in runs of kRun keys into bkey0,
-// four waves per run (kSortE keys per thread: a quarter of the network's
+// aabb.cu:589-611, thrust_helper.cu:21-29) in runs of at most kRun keys into
+// bkey0, four waves per run (kSortE keys per thread: a quarter of the network's
 // instructions per wave of a one-wave run, for three LDS stages); the
 // remaining blocks count the survivors of each window tile.
-constexpr int kRun = 512;                                // keys per sorted run of the stride
+constexpr int kRun = 512;                                // most keys of a sorted run of the stride
 constexpr int kSortE = 2;                                // keys per thread
-constexpr int kSortRunThreads = kRun / kSortE;           // 256: four waves per run
-constexpr int kSortBlockKeys = kTileThreads * kSortE;    // 512: one run per block
-constexpr int kSortParts = kTile / kSortBlockKeys;       // blocks per stride tile
+constexpr int kSortParts = kTile / kRun;                 // blocks per stride tile, a run each
+static_assert(kRun == kSortE * kTileThreads, "");
+constexpr int kRunChunks = kRun / 64;
+typedef uint64_t KeyPair __attribute__((ext_vector_type(2)));
+
+// The runs of a stride of SS keys: as few as hold it, of equal length but for
+// one key (a short last run's 64 keys would span all other runs, whose every
+// chunk the rank kernel would then search).
+struct Runs {
+    int n, len, longer;  // runs; keys of a run, and how many of the first hold one more
+    __device__ __forceinline__ Runs(int SS) : n((SS + kRun - 1) / kRun), len(SS / n), longer(SS - n * len) {}
+    __device__ __forceinline__ int start(int r) const { return r * len + min(r, longer); }
+};
 
 __global__ __launch_bounds__(kTileThreads) void k_sort_expire(BatchArgs a) {
     __shared__ uint64_t lds[kTile];
@@ -498,20 +508,24 @@ __global__ __launch_bounds__(kTileThreads) void k_sort_expire(BatchArgs a) {
     const StreamDev &S = a.s[s];
     const IO io = a.use_io1 ? a.io1 : a.io[s];
     const int SS = ldc(S.S);
-    const int tile0 = (gt - ldc(a.pre_stile[s])) * kTile + (g % kSortParts) * kSortBlockKeys;
-    if (tile0 >= SS) return;  // the whole block: past the stride's end
-    const int r = threadIdx.x / kSortRunThreads, t = threadIdx.x % kSortRunThreads;
+    const Runs runs(SS);
+    const int run = (gt - ldc(a.pre_stile[s])) * kSortParts + g % kSortParts;
+    if (run >= runs.n) return;  // the whole block: past the stride's end
+    const int start = runs.start(run), nvalid = runs.start(run + 1) - start;
     uint64_t v[kSortE];
-    sort_tile_keys<kRun, kSortE>(key_grid(S), gl(io.in), SS, tile0 + r * kRun, ldc(ldc(S.mut)->u) * SS, v,
-                                 lds + r * kRun, t);
+    sort_tile_keys<kRun, kSortE>(key_grid(S), gl(io.in), start + nvalid, start, ldc(ldc(S.mut)->u) * SS, v, lds,
+                                 threadIdx.x);
     // coalesced store through LDS (thread i holds positions kSortE * i ..)
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < kSortE; e++) lds[threadIdx.x * kSortE + e] = v[e];
     __syncthreads();
-    const int nvalid = min(kSortBlockKeys, SS - tile0);
     const gptr<uint64_t> bkey0 = gl(ldc(S.bkey0));
-    for (int i = threadIdx.x; i < nvalid; i += kTileThreads) bkey0[tile0 + i] = lds[i];
+    for (int i = threadIdx.x; i < nvalid; i += kTileThreads) bkey0[start + i] = lds[i];
+    // first and last key of every 64
+    if (threadIdx.x < kRunChunks && (int)threadIdx.x * 64 < nvalid)
+        gl((KeyPair *)ldc(S.bends))[run * kRunChunks + threadIdx.x] =
+            KeyPair{lds[threadIdx.x * 64], lds[min((int)threadIdx.x * 64 + 63, nvalid - 1)]};
 }
 
 // Ordered compaction of the survivors into the A arrays. Each tile's offset
@@ -564,27 +578,42 @@ __device__ __forceinline__ void expire_compact(const BatchArgs &a, int g, int *l
     }
 }
 
+// LDS written by lanes of this wave is read by others next.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Launch 2 of a slide: blocks [0, rank_blocks) place each stride key at its rank
 // in the whole stride - its index in its sorted run plus, for every other
 // run, the number of that run's keys below it - and write keys and
-// coordinates to the B1 arrays: the stride sorted by (cell, slot). The other
-// runs are staged in LDS kStageRuns at a time (the next ones load while the
-// current ones are searched). With SPLIT == 1 a block ranks 256 keys, one per
-// thread, and every thread searches every staged run. With SPLIT == 4 a
-// block ranks 64 keys and its four waves split each stage's runs between
-// them, summing their partial ranks in LDS at the end: four times the blocks
-// and a quarter of the searches per thread, for strides too small to fill the
-// device with 256-key blocks. The blocks after them compact the window's
-// survivors (expire_compact), which depends on the same launch before.
-constexpr int kStageRuns = 8;  // 32 KB of LDS
+// coordinates to the B1 arrays: the stride sorted by (cell, slot). The blocks
+// after them compact the window's survivors (expire_compact), which depends on
+// the same launch before.
+//
+// 64 consecutive keys of a run lie close together, so of another run's chunks
+// of 64 keys nearly all are wholly below or wholly above them: the chunks'
+// first and last keys (written by the sort) tell, one chunk per lane. Only the
+// two or so chunks of each run that reach into the keys' span are loaded into
+// LDS and searched, kRankChunks at a time, the next ones on their way
+// meanwhile. What bounds it is the searches: seven dependent LDS reads per
+// chunk and key, S / 512 runs of two chunks. Searching whole runs staged in
+// LDS, as before, moved the whole stride through every block; us of the launch
+// so and now: 20,501 keys 17.0 and 11.8, 50,000 keys 48 and 27.5, 10,000 keys
+// 10.4 and 6.8, the 64-stream batch (321,000 keys) 57 and 42.5, of which the
+// compaction takes about 20. Eight chunks a step: 12.4 and 31.6 us at 20,501
+// and 50,000 keys; three probes a step 11.2 and 28.1. With SPLIT == 1 each wave ranks 64 keys by itself; with
+// SPLIT == 4 the four waves of a block split the other runs between them,
+// summing their partial ranks in LDS at the end, for strides too small to fill
+// the device otherwise.
+constexpr int kRankChunks = 4;  // chunks searched together
 
 template <int SPLIT>
 __global__ __launch_bounds__(kTileThreads) void k_rank(BatchArgs a, int rank_blocks) {
     constexpr int kWaves = kTileThreads / 64;
-    constexpr int kKeys = kTileThreads / SPLIT;  // keys per block, all in one run (kKeys divides kRun)
-    constexpr int kParts = kTile / kKeys;        // blocks per stride tile
-    constexpr int kMine = kStageRuns / SPLIT;    // staged runs each thread searches
-    __shared__ uint64_t lds[kStageRuns * kRun];
+    constexpr int kParts = kTile / 64 / (kWaves / SPLIT);  // blocks per stride tile
+    __shared__ uint64_t lds[kWaves][kRankChunks][64];
     __shared__ int part[SPLIT > 1 ? kWaves : 1][64];
     if ((int)blockIdx.x >= rank_blocks) {  // the survivor compaction shares the launch
         expire_compact(a, blockIdx.x - rank_blocks, (int *)part);
@@ -594,34 +623,25 @@ __global__ __launch_bounds__(kTileThreads) void k_rank(BatchArgs a, int rank_blo
     const int gb = g / kParts;
     const int s = find_stream_c(a.pre_stile, a.n, gb);
     const StreamDev &S = a.s[s];
-    // the stream's fields as constant memory and its arrays as global memory:
-    // global loads wait on their own counter, so the next stage's keys load
-    // while the LDS searches of this stage run
     const int SS = ldc(S.S), dim = ldc(S.dim);
-    const int i0 = (gb - ldc(a.pre_stile[s])) * kTile + (g % kParts) * kKeys;
-    if (i0 >= SS) return;  // the whole block: past the stride's end
+    const int wv = uni(threadIdx.x >> 6), lane = lane_id();
+    const int sigma = wv % SPLIT;  // which of the other runs this wave searches
+    const Runs runs(SS);
+    // this wave's or block's 64 keys: a chunk of a run
+    const int mine = ((gb - ldc(a.pre_stile[s])) * kParts + g % kParts) * (kWaves / SPLIT) + (SPLIT > 1 ? 0 : wv);
+    const int myrun = mine / kRunChunks;
+    const int i0 = runs.start(myrun) + mine % kRunChunks * 64;
+    const int nk = min(runs.start(myrun + 1) - i0, 64);
+    if (myrun >= runs.n || nk <= 0) return;  // past the stride's or the run's end (the whole block where its waves meet)
     const gptr<const uint64_t> bkey0 = gl((const uint64_t *)ldc(S.bkey0));
-    const int wv = threadIdx.x >> 6, lane = lane_id();
-    const int sigma = wv % SPLIT;  // which of each stage's runs this wave searches
-    const int i = i0 + (SPLIT > 1 ? lane : (int)threadIdx.x);
-    const bool valid = i < SS;
+    const gptr<const KeyPair> bends = gl((const KeyPair *)ldc(S.bends));
+    const int i = i0 + lane;
+    const bool valid = lane < nk;
     const uint64_t key = valid ? bkey0[i] : ~0ull;
-    const int myrun = i0 / kRun, nr = (SS + kRun - 1) / kRun;
-    constexpr int per = kStageRuns * kRun / kTileThreads;
-    auto run_of = [&](int o) { return o < myrun ? o : o + 1; };  // the o-th run other than the block's
-    // keys of the staged runs o0 .. o0 + kStageRuns - 1, ~0 past their ends
-    auto load_stage = [&](int o0, uint64_t(&st)[per]) {
-#pragma unroll
-        for (int e = 0; e < per; e++) {
-            const int slot = threadIdx.x + e * kTileThreads;  // [0, kStageRuns * kRun)
-            const int q = slot / kRun, j = slot % kRun;
-            const int o = o0 + q;
-            const int r = run_of(o);
-            st[e] = (o < nr - 1 && j < min(kRun, SS - r * kRun)) ? bkey0[r * kRun + j] : ~0ull;
-        }
-    };
-    uint64_t cur[per], nxt[per];
-    if (nr > 1) load_stage(0, cur);
+    // this lane's chunk among those of 8 runs, whose first is r0
+    auto run_of = [&](int r0) { return r0 + (lane >> 3) * SPLIT; };
+    auto ends_of = [&](int r0) { return bends[min(run_of(r0), runs.n - 1) * kRunChunks + (lane & 7)]; };
+    KeyPair ends = ends_of(sigma);
     // the point's coordinates are needed only at the end: loaded now
     const IO io = a.use_io1 ? a.io1 : a.io[s];
     float px = 0.f, py = 0.f, pz = 0.f;
@@ -632,39 +652,48 @@ __global__ __launch_bounds__(kTileThreads) void k_rank(BatchArgs a, int rank_blo
         py = dim > 1 ? p[1] : 0.f;
         pz = dim > 2 ? p[2] : 0.f;
     }
-    int rank = 0;
-    for (int o0 = 0; o0 < nr - 1; o0 += kStageRuns) {
-        const bool more = o0 + kStageRuns < nr - 1;
-        if (more) load_stage(o0 + kStageRuns, nxt);
-        int len[kMine];
+    const uint64_t kmin = readlane64(key, 0), kmax = readlane64(key, nk - 1);
+    int rank = 0, whole = 0;
+    for (int r0 = sigma; r0 < runs.n; r0 += 8 * SPLIT) {
+        const int r = run_of(r0);
+        const int left = r < runs.n && r != myrun ? runs.start(r + 1) - runs.start(r) - (lane & 7) * 64 : 0;
+        const bool below = left > 0 && ends.y < kmin;
+        whole += below ? min(left, 64) : 0;
+        uint64_t m = __ballot(left > 0 && !below && ends.x < kmax);
+        if (r0 + 8 * SPLIT < runs.n) ends = ends_of(r0 + 8 * SPLIT);
+        // the next chunks' keys; every load is issued, clamped, so that no
+        // branch waits for it
+        uint64_t v[kRankChunks];
+        int n[kRankChunks];
+        auto load = [&]() {
 #pragma unroll
-        for (int q = 0; q < kMine; q++) {
-            const int o = o0 + q * SPLIT + sigma;
-            len[q] = o < nr - 1 ? min(kRun, SS - run_of(o) * kRun) : 0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < per; e++) lds[threadIdx.x + e * kTileThreads] = cur[e];
-        __syncthreads();
-        int pos[kMine];
-#pragma unroll
-        for (int q = 0; q < kMine; q++) pos[q] = 0;
-#pragma unroll
-        for (int step = kRun; step > 0; step >>= 1) {
-#pragma unroll
-            for (int q = 0; q < kMine; q++) {
-                const int probe = pos[q] + step;
-                const uint64_t v = lds[(q * SPLIT + sigma) * kRun + min(probe, kRun) - 1];
-                if (probe <= len[q] && v < key) pos[q] = probe;
+            for (int q = 0; q < kRankChunks; q++) {
+                const int l = m ? __ffsll((unsigned long long)m) - 1 : 0;
+                const int r1 = r0 + (l >> 3) * SPLIT, p0 = runs.start(r1) + (l & 7) * 64;
+                n[q] = m ? runs.start(r1 + 1) - p0 : 0;
+                v[q] = bkey0[min(p0 + lane, SS - 1)];
+                m &= m - 1ull;
             }
-        }
+        };
+        load();
+        while (n[0] > 0) {
 #pragma unroll
-        for (int q = 0; q < kMine; q++) rank += pos[q];
-        if (more) {
+            for (int q = 0; q < kRankChunks; q++) lds[wv][q][lane] = lane < n[q] ? v[q] : ~0ull;
+            load();
+            wave_sync();
+            int pos[kRankChunks] = {};
 #pragma unroll
-            for (int e = 0; e < per; e++) cur[e] = nxt[e];
+            for (int step = 32; step > 0; step >>= 1) {
+#pragma unroll
+                for (int q = 0; q < kRankChunks; q++)
+                    pos[q] += lds[wv][q][pos[q] + step - 1] < key ? step : 0;
+            }
+#pragma unroll
+            for (int q = 0; q < kRankChunks; q++) rank += pos[q] + (lds[wv][q][pos[q]] < key ? 1 : 0);
+            wave_sync();
         }
     }
+    rank += wave_sum(whole);
     if (SPLIT > 1) {
         part[wv][lane] = rank;
         __syncthreads();
@@ -673,13 +702,12 @@ __global__ __launch_bounds__(kTileThreads) void k_rank(BatchArgs a, int rank_blo
         for (int w = 1; w < SPLIT; w++) rank += part[w][lane];
     }
     if (!valid) return;
-    rank += i - myrun * kRun;
+    rank += i - runs.start(myrun);
     gl(S.bkey1)[rank] = key;
     gl(S.bx1)[rank] = px;
     if (dim > 1) gl(S.by1)[rank] = py;
     if (dim > 2) gl(S.bz1)[rank] = pz;
 }
-
 
 // Number of elements of A among the first d of merge(A, B); keys are unique.
 // P(i) = A[i] < B[d-1-i] holds exactly for i below the answer. One wave
@@ -2084,13 +2112,6 @@ __device__ __forceinline__ uint64_t from_lane64(uint64_t v, int l) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-// LDS written by lanes of this wave is read by others next.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // First and last cell before cell A of stencil row r (Bf > Bl: none).
 __device__ __forceinline__ void row_cells(const CellView &V, int A, uint64_t rw, int *Bf, int *Bl) {
     const int rx = (int)(uint32_t)rw, ry = (int)(uint32_t)(rw >> 32);
@@ -2228,6 +2249,7 @@ __device__ __forceinline__ void link_tile(const CellView &V, int k, int c0, int 
 constexpr int kPairCap = 512;  // 64 rows of at most kRowCells cells, and fewer than 64 pairs left over
 constexpr int kFew = 4;  // points of a cell tested in a lane
 constexpr int kRowCells = 2 * kMaxK + 1;  // most cells of a stencil row
+static_assert(64 * kRowCells + 63 <= kPairCap, "");
 
 struct PairBuf {
     uint32_t *e;  // this wave's LDS slice
