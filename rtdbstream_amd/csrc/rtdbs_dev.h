@@ -64,6 +64,7 @@ struct IO {
 struct StreamDev {
     int32_t dim, W, S, min_pts;
     int32_t k, R, slot_bits, units;
+    int32_t row_w, row_div;  // stencil rows stored together per cell, and 256 / row_w + 1 (RowTable)
     int32_t dense_ok;  // side eps/k with k*k > dim: points of one interior cell are within eps
     float eps2;        // fl32(eps*eps)
     double inv_side;

@@ -233,6 +233,8 @@ extern "C" int rtdbs_stream_create(const rtdbs_params *params, rtdbs_stream **ou
     D.min_pts = s->p.min_pts;
     D.k = s->k;
     D.R = s->R;
+    D.row_w = s->p.dim == 3 ? 2 * s->k + 1 : s->R;
+    D.row_div = 256 / D.row_w + 1;
     D.slot_bits = s->slot_bits;
     D.units = s->p.window / s->p.stride;
     D.dense_ok = s->dense_ok;
