@@ -333,7 +333,8 @@ typedef struct {
     int64_t count_queries; /* points whose neighbours were counted (rays of the core pass) */
     int64_t count_tests;   /* distance tests of the range count (intersections; num_dist_calculations) */
     int64_t merge_tests;   /* distance tests of the cluster merge (cluster-pass intersections) */
-    int64_t border_tests;  /* distance tests of the border pass */
+    int64_t border_tests;  /* distance tests of the border pass (with the counters on every non-core point
+                              is walked, those whose count found no neighbour too) */
     int64_t unites;        /* union-find unite calls */
     int64_t merge_pairs;   /* touching element pairs found by the merge */
     int32_t cell_parallel; /* 1: count and border ran cell-parallel; 0: either ran point-parallel (large

@@ -42,6 +42,7 @@ enum Stat {
 
 constexpr uint8_t kFlagCore = 1;
 constexpr uint8_t kFlagDense = 2;
+constexpr uint8_t kFlagAlone = 4;  // no other point within eps (set where the count found that out)
 constexpr uint8_t kCellSafe = 1;
 constexpr uint8_t kCellDense = 2;
 constexpr int kNoCore = 0x7fffffff;  // fcore of a cell without cores
@@ -90,7 +91,7 @@ struct StreamDev {
     uint8_t *cflag;   // W: kCellSafe | kCellDense per cell
     int32_t *fcore;   // W: first (minimum-slot) core position of each cell, kNoCore if none
     // clustering
-    uint8_t *flags;   // W: kFlagCore | kFlagDense
+    uint8_t *flags;   // W: kFlagCore | kFlagDense, or kFlagAlone
     uint64_t *uf;     // 2W: union-find entries of cells [0, W) and of unsafe cells' cores, W + position
     int32_t *tile_a;  // ceil(W/kWTile): survivors per tile
     int32_t *tile_b;  // ceil(W/kWTile): cell starts per tile
