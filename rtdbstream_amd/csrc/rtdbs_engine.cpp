@@ -132,8 +132,8 @@ static Layout make_layout(const rtdbs_params &p, int R) {
     L.off_mut = take(sizeof(StreamMut));
     L.off_skey = take(W * 8);
     // window coordinates (both buffers of the ping-pong) with kCandPad
-    // readable floats past the end, a margin: the candidate walks read real
-    // candidates only
+    // readable floats past the end: the candidate walks load four at a time
+    // from a row's candidates
     const size_t wc = (W + kCandPad) * 4;
     L.off_sx = take(wc);
     L.off_sy = d > 1 ? take(wc) : 0;

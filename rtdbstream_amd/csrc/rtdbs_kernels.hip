@@ -2688,25 +2688,74 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_merge_cells(BatchArgs a) {
 // adjacent and read the same candidates. D is the stream's dimension, so the
 // distance test and the loads carry no per-candidate dimension selects.
 //
-// Flat walks: a lane's rows, a group at a time, walked as one sequence of
-// candidates. The group's row words come in one round trip, then kFlat
-// candidates per round trip whatever the rows' lengths, so that a row holding
-// a cell or two does not cost a round trip of its own. Candidate t of a group
-// lies in the last row i with pre[i] <= t (pre: the candidates of the group's
+// Walks by fours: a lane's rows, a group at a time, walked as one sequence of
+// fours, each up to four candidates of one row by one 16-byte load per axis,
+// kFours of them per round trip whatever the rows' lengths. Four t of a group
+// lies in the last row i with pre[i] <= t (pre: the fours of the group's
 // earlier rows; an empty row shares its pre with the next row, which
-// overrides it), at position t + base[i].
+// overrides it) and starts at position base[i] + 4 * t; past the row's end it
+// reads other candidates or up to three words past the window, which the
+// coordinate arrays hold (kCandPad), and leaves them out.
 //
-// What bounds the count is its vector loads (7.5 M a launch of 64 streams, some
-// 13 cycles of a CU each), so the second half of a round trip's is left out
-// where no lane of the wave has that many candidates: 64 streams 164 -> 152 us,
-// 24 served streams 86 -> 83. Asked before every pair of candidates: 155 us,
-// before every one: 160; rounds of 12 asked every four: 158. The outputs' walks
-// gain nothing by it.
-constexpr int kFlat = 8;        // candidates per round trip of a flat walk
+// What bounds the walks is the work per candidate: finding its row and an
+// address and a load per axis were 16 instructions of 26 when each candidate
+// was found by itself, eight a round trip. A row of one or two cells fills half
+// its fours, and still a four costs less than its candidates did. Count so and
+// by fours: 64 streams 152 and 121 us, 24 served streams 82 and 56; outputs 137
+// and 113, 71 and 72, one million points 76 and 73. One, three and four fours a
+// round trip in the count: 137, 126 and 129 us at 64 streams; groups of 3, 4
+// and 8 rows: 135, 128 and 125.
+typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int kFours = 2;
 constexpr int kBorderRows = 8;  // rows per group of the outputs' walk (no early exit)
 
+// The fours of a group of N rows, of `first + i * step`; past the last row none.
+template <int N>
+struct FourWalk {
+    int base[N], pre[N], end[N];
+    int n = 0;  // fours
+    __device__ __forceinline__ FourWalk(const CellView &V, gptr<const uint64_t> rows, int first, int step) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int r = first + i * step;
+            const uint64_t rw = r < V.R ? rows[V.rows.row(r)] : 0ull;
+            const int rx = (int)(uint32_t)rw, ry = (int)(uint32_t)(rw >> 32);  // rx < ry, or both 0
+            pre[i] = n;
+            base[i] = rx - 4 * n;
+            end[i] = ry;
+            n += (ry - rx + 3) >> 2;
+        }
+    }
+    // First position of four t, and how many candidates there are from it to
+    // its row's end; past the last four (n > 0) the last one's, and none.
+    __device__ __forceinline__ void at(int t, int *pos, int *left) const {
+        const int tt = min(t, n - 1);
+        int b = base[0], e = end[0];
+#pragma unroll
+        for (int i = 1; i < N; i++) {
+            b = tt >= pre[i] ? base[i] : b;
+            e = tt >= pre[i] ? end[i] : e;
+        }
+        *pos = b + 4 * tt;
+        *left = t < n ? e - *pos : 0;
+    }
+};
+
+template <int D>
+struct Four {
+    F4 x, y, z;
+    __device__ __forceinline__ void load(const CellView &V, int pos) {
+        x = *(gptr<const F4>)(V.sx + pos);
+        if (D > 1) y = *(gptr<const F4>)(V.sy + pos);
+        if (D > 2) z = *(gptr<const F4>)(V.sz + pos);
+    }
+    __device__ __forceinline__ float sqd_to(int v, float qx, float qy, float qz) const {
+        return sqd(D, qx, qy, qz, x[v], D > 1 ? y[v] : 0.f, D > 2 ? z[v] : 0.f);
+    }
+};
+
 // One lane's share of a query's stencil: rows first, first + step, ..., in
-// flat groups of kRowGroup rows, nearest rows first. The count is checked
+// groups of kRowGroup rows, nearest rows first. The count is checked
 // against min_pts once per round trip.
 template <int D>
 __device__ __forceinline__ int count_walk(const CellView &V, int c, float qx, float qy, float qz, int first,
@@ -2716,35 +2765,22 @@ __device__ __forceinline__ int count_walk(const CellView &V, int c, float qx, fl
     int cnt = 0;
     const gptr<const uint64_t> rows = V.rows.of(c);
     for (int r0 = first; r0 < V.R; r0 += kRowGroup * step) {
-        int base[kRowGroup], pre[kRowGroup];
-        int T = 0;
+        const FourWalk<kRowGroup> w(V, rows, r0, step);
+        for (int t0 = 0; t0 < w.n; t0 += kFours) {
+            Four<D> f[kFours];
+            int left[kFours];
 #pragma unroll
-        for (int i = 0; i < kRowGroup; i++) {
-            const uint64_t rw = (r0 + i * step < V.R) ? rows[V.rows.row(r0 + i * step)] : 0ull;
-            const int rx = (int)(uint32_t)rw, ry = (int)(uint32_t)(rw >> 32);  // rx < ry, or both 0
-            pre[i] = T;
-            base[i] = rx - T;
-            T += ry - rx;
-        }
-        for (int t0 = 0; t0 < T; t0 += kFlat) {
-            float cx[kFlat], cy[kFlat], cz[kFlat];
-#pragma unroll
-            for (int u = 0; u < kFlat; u++) {
-                if (u == kFlat / 2 && !__any(T - t0 > u)) break;
-                // clamped to the last candidate: every load reads a real one
-                const int t = min(t0 + u, T - 1);
-                int b = base[0];
-#pragma unroll
-                for (int i = 1; i < kRowGroup; i++) b = t >= pre[i] ? base[i] : b;
-                const uint32_t o = (uint32_t)(t + b) << 2;
-                cx[u] = ldo(V.sx, o);
-                cy[u] = D > 1 ? ldo(V.sy, o) : 0.f;
-                cz[u] = D > 2 ? ldo(V.sz, o) : 0.f;
+            for (int u = 0; u < kFours; u++) {
+                int pos;
+                w.at(t0 + u, &pos, &left[u]);
+                f[u].load(V, pos);
             }
-            const int nv = T - t0;
-            tests += min(nv, kFlat);
 #pragma unroll
-            for (int u = 0; u < kFlat; u++) cnt += (u < nv) & (sqd(D, qx, qy, qz, cx[u], cy[u], cz[u]) < e2);
+            for (int u = 0; u < kFours; u++) {
+                tests += min(left[u], 4);
+#pragma unroll
+                for (int v = 0; v < 4; v++) cnt += (v < left[u]) & (f[u].sqd_to(v, qx, qy, qz) < e2);
+            }
             if (cnt >= minpts) return cnt;
         }
     }
@@ -2812,7 +2848,7 @@ __global__ __launch_bounds__(64) void k_count_points(BatchArgs a) {
 // stream's ring cursor, as the cell-parallel output kernel does. D is the
 // stream's dimension.
 //
-// One lane's share of a non-core point's stencil in flat groups of
+// One lane's share of a non-core point's stencil in groups of
 // kBorderRows rows (larger than the count's: no early exit here), without an
 // early exit: the minimum root of the cores within eps. A candidate's flags
 // and cell load only when it is within eps, and the cell's root only when it is
@@ -2825,45 +2861,32 @@ __device__ __forceinline__ int border_walk(const CellView &V, int c, float qx, f
     int best = INT_MAX, seen = -1;
     const gptr<const uint64_t> rows = V.rows.of(c);
     for (int r0 = first; r0 < V.R; r0 += kBorderRows * step) {
-        int base[kBorderRows], pre[kBorderRows];
-        int T = 0;
+        const FourWalk<kBorderRows> w(V, rows, r0, step);
+        for (int t0 = 0; t0 < w.n; t0 += kFours) {
+            Four<D> f[kFours];
+            int pos[kFours], left[kFours];
 #pragma unroll
-        for (int i = 0; i < kBorderRows; i++) {
-            const uint64_t rw = (r0 + i * step < V.R) ? rows[V.rows.row(r0 + i * step)] : 0ull;
-            const int rx = (int)(uint32_t)rw, ry = (int)(uint32_t)(rw >> 32);
-            pre[i] = T;
-            base[i] = rx - T;
-            T += ry - rx;
-        }
-        for (int t0 = 0; t0 < T; t0 += kFlat) {
-            float cx[kFlat], cy[kFlat], cz[kFlat];
-            int pos[kFlat];
-#pragma unroll
-            for (int u = 0; u < kFlat; u++) {
-                const int t = min(t0 + u, T - 1);
-                int b = base[0];
-#pragma unroll
-                for (int i = 1; i < kBorderRows; i++) b = t >= pre[i] ? base[i] : b;
-                pos[u] = t + b;
-                const uint32_t o = (uint32_t)pos[u] << 2;
-                cx[u] = ldo(V.sx, o);
-                cy[u] = D > 1 ? ldo(V.sy, o) : 0.f;
-                cz[u] = D > 2 ? ldo(V.sz, o) : 0.f;
+            for (int u = 0; u < kFours; u++) {
+                w.at(t0 + u, &pos[u], &left[u]);
+                f[u].load(V, pos[u]);
             }
-            const int nv = T - t0;
-            tests += min(nv, kFlat);
 #pragma unroll
-            for (int u = 0; u < kFlat; u++)
-                if ((u < nv) & (sqd(D, qx, qy, qz, cx[u], cy[u], cz[u]) < e2)) {
-                    const int f = ldo(V.flags, (uint32_t)pos[u]);
-                    const int pc = ldo(V.pcell, (uint32_t)pos[u] << 2);
-                    arrived(pc);
-                    if ((f & kFlagCore) && pc != seen) {
-                        const uint64_t e = V.uf[pc];
-                        if (e != kUfUnsafe) seen = pc;
-                        best = min(best, core_cid(V, e, pos[u]));
+            for (int u = 0; u < kFours; u++) {
+                tests += min(left[u], 4);
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if ((v < left[u]) & (f[u].sqd_to(v, qx, qy, qz) < e2)) {
+                        const int p = pos[u] + v;
+                        const int fl = ldo(V.flags, (uint32_t)p);
+                        const int pc = ldo(V.pcell, (uint32_t)p << 2);
+                        arrived(pc);
+                        if ((fl & kFlagCore) && pc != seen) {
+                            const uint64_t e = V.uf[pc];
+                            if (e != kUfUnsafe) seen = pc;
+                            best = min(best, core_cid(V, e, p));
+                        }
                     }
-                }
+            }
         }
     }
     return best;
