@@ -600,8 +600,11 @@ static int env_int(const char *name, int def, int lo, int hi) {
 // Windows up to this many points in one launch use the cell-parallel count of
 // a single stream, and the launch sizes of a latency-bound launch.
 constexpr long long kCellParMaxPoints = 1000000;
-// The same for the cell-parallel outputs, and the count of several streams.
-constexpr long long kCellParMaxShared = 250000;
+// The same for the count of several streams, and for the outputs of one stream
+// and of several.
+constexpr long long kCellCountShared = 60000;
+constexpr long long kCellOutputsOne = 80000;
+constexpr long long kCellOutputsShared = 110000;
 
 // Uploads descriptors and prefix tables; drops a captured graph. Called when
 // the batch is built and whenever a member stream was re-initialised.
@@ -659,24 +662,25 @@ int refresh_batch(rtdbs_batch *b) {
     b->shape.rows_blocks = (int)std::max(1ll, std::min((long long)device_cus() * rcap, pb));
     // Count and outputs: cell-parallel (coalesced candidate loads, a wave per
     // cell) while a launch is small and latency-bound, point-parallel once its
-    // windows fill the device's lanes. A batch of several streams switches both
-    // above kCellParMaxShared points (us cell / point: 338,000 points of 16
-    // streams count 56 / 50, outputs 58 / 46; 687,000 of 32 streams 89 / 62, 103 /
-    // 60; 110,000 of 8 streams 23 / 19, 24 / 38). A single stream's outputs switch
-    // there too (500,000 3-D points 53 / 43, 1-D 33 / 12; 100,000 13 / 18), its
-    // count only above kCellParMaxPoints (500,000 points 45 / 73, 1 M 121 / 183).
+    // windows fill the device's lanes. us cell / point (the point count with the
+    // pass over the cells that follows it): several streams count 36,000 points
+    // 11.6 / 12.5, 91,000 20.6 / 16.9, 338,000 59 / 38; outputs 91,000 20.4 / 23.7,
+    // 125,000 26.2 / 24.5, 338,000 58 / 33. One stream's outputs: 61,500 3-D
+    // points 9.7 / 12.5, 100,000 12.6 / 11.1 and 10.7 / 4.7 in 1-D, 14.0 / 13.1 in
+    // 2-D, 500,000 54 / 29; its count only above kCellParMaxPoints (200,000 3-D
+    // points 23.5 / 29.2, 500,000 48 / 56, one million uneven ones 123 / 116).
     // RTDBS_NEIGHBOR_MODE: 1 forces cell-parallel, 2 point-parallel (over a
     // single stream's own neighbor_mode).
     const int nmode = env_int("RTDBS_NEIGHBOR_MODE", 0, 0, 2);
     const int pmode = n == 1 ? b->streams[0]->p.neighbor_mode : 0;  // a single stream's own setting
     const int mode = nmode ? nmode : pmode;
-    b->shape.cellpar = mode == 1 || (mode == 0 && cells_total <= kCellParMaxShared);
+    b->shape.cellpar = mode == 1 || (mode == 0 && cells_total <= (n == 1 ? kCellOutputsOne : kCellOutputsShared));
     // the range count's own form (RTDBS_COUNT_MODE: 1 cell-parallel, 2
     // point-parallel; otherwise as above)
     const int cmode = env_int("RTDBS_COUNT_MODE", 0, 0, 2);
     b->shape.count_cell =
         cmode ? (cmode == 1)
-              : mode == 1 || (mode == 0 && cells_total <= (n == 1 ? kCellParMaxPoints : kCellParMaxShared));
+              : mode == 1 || (mode == 0 && cells_total <= (n == 1 ? kCellParMaxPoints : kCellCountShared));
     // cell-parallel grid: 16 blocks per CU while the launch is small; 32 for
     // large batches, where it carries the merge alone (64 streams: 455 ->
     // ~400 us). RTDBS_CELLPAR_PER_CU overrides.
