@@ -509,7 +509,7 @@ static int batch_alloc(rtdbs_batch *b) {
     b->d_io = (IO *)(b->dmem + desc_b);
     b->d_pre = (int32_t *)(b->dmem + desc_b + io_b);
     b->d_stats = (unsigned long long *)(b->dmem + desc_b + io_b + pre_b);
-    HIPCHK(hipHostMalloc((void **)&b->hmem, desc_b + io_b + pre_b + sizeof(FirstWindow), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void **)&b->hmem, desc_b + io_b + pre_b + sizeof(FirstWindow), hipHostMallocCoherent));
     b->h_desc = (StreamDev *)b->hmem;
     b->h_io = (IO *)(b->hmem + desc_b);
     b->h_pre = (int32_t *)(b->hmem + desc_b + io_b);
@@ -925,7 +925,7 @@ static int enqueue_copies(const std::vector<Copy> &v, hipMemcpyKind kind, CopySe
         fit = fit && (((uintptr_t)c.dst | (uintptr_t)c.src | c.bytes) & 3) == 0;
         words += c.bytes / 4;
     }
-    if (fit && words < (size_t(1) << 32)) {
+    if (fit && words < (size_t(1) << 31)) {  // (the kernel counts words in 32 bits)
         uint32_t first = 0;
         for (size_t i = 0; i < v.size(); i++) {
             list[i] = CopySeg{v[i].src, v[i].dst, first, (uint32_t)(v[i].bytes / 4)};
@@ -978,7 +978,7 @@ static int ensure_xfer(rtdbs_batch *b) {
         b->h_stage = nullptr;
         b->h_stage_bytes = 0;
         const size_t want = b->solo ? total : grow;
-        hipError_t e = hipHostMalloc((void **)&b->h_stage, want, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void **)&b->h_stage, want, hipHostMallocCoherent);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return fail(RTDBS_ENOMEM, "pinned staging of %zu bytes: %s", want, hipGetErrorString(e));
@@ -1410,7 +1410,9 @@ extern "C" int rtdbs_host_alloc(size_t bytes, void **ptr) {
     if (!ptr) return fail(RTDBS_EINVAL, "ptr is NULL");
     *ptr = nullptr;
     if (bytes == 0) bytes = 1;
-    hipError_t e = hipHostMalloc(ptr, bytes, hipHostMallocDefault);
+    // coherent whatever the process's default: kernels read and write these
+    // buffers while others of the same stream still run
+    hipError_t e = hipHostMalloc(ptr, bytes, hipHostMallocCoherent);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *ptr = nullptr;
