@@ -42,6 +42,7 @@ enum Stat {
 
 constexpr uint8_t kFlagCore = 1;
 constexpr uint8_t kFlagDense = 2;
+constexpr uint8_t kFlagLoose = 8;  // a core of an unsafe cell, an element of its own
 constexpr uint8_t kFlagAlone = 4;  // no other point within eps (set where the count found that out)
 constexpr uint8_t kCellSafe = 1;
 constexpr uint8_t kCellDense = 2;
@@ -91,7 +92,7 @@ struct StreamDev {
     uint8_t *cflag;   // W: kCellSafe | kCellDense per cell
     int32_t *fcore;   // W: first (minimum-slot) core position of each cell, kNoCore if none
     // clustering
-    uint8_t *flags;   // W: kFlagCore | kFlagDense, or kFlagAlone
+    uint8_t *flags;   // W: kFlagCore | kFlagDense, kFlagCore | kFlagLoose or kFlagAlone
     uint64_t *uf;     // 2W: union-find entries of cells [0, W) and of unsafe cells' cores, W + position
     int32_t *tile_a;  // ceil(W/kWTile): survivors per tile
     int32_t *tile_b;  // ceil(W/kWTile): cell starts per tile
@@ -110,6 +111,7 @@ struct BatchArgs {
     int32_t *cell_pre;         // n+1 prefix of cells per stream (written by k_rows)
     int32_t *ctile_pre;        // n+1 prefix of cell tiles (cell_tile cells each) per stream (written by k_rows)
     int32_t cell_tile;         // cells per wave item of the merge of safe cells, 1..64
+    int32_t wave_merge;        // 1: every stream's cells are merged by a wave each (k_union)
     int32_t xcd_groups;        // kXcd* bits: kernels whose XCDs each take one contiguous range of work
 };
 
@@ -129,8 +131,8 @@ struct LaunchShape {
     int32_t cellpar_blocks;  // blocks of the cell-parallel count and border kernels
     int32_t cellpar;         // 1: cell-parallel output kernel, 0: point-parallel
     int32_t count_cell;      // 1: cell-parallel range count (writes fcore and rep), 0: point-parallel
-    int32_t link;            // 1: some stream has safe cells: merged by k_merge_cells
-    int32_t unsafe;          // 1: some stream has none (reach 1): merged by k_union
+    int32_t link;            // 1: some stream is merged by k_merge_cells
+    int32_t by_wave;         // 1: some stream is merged by k_union
     int32_t link_blocks;     // blocks of k_merge_cells and k_cell_cores
     int32_t small_update;    // window positions per thread of the one-block update in LDS (k_update_small), 0: not used
     int32_t rank_split;      // 1: stride rank with 64-key blocks (small strides), 0: 256-key blocks

@@ -603,8 +603,14 @@ constexpr long long kCellParMaxPoints = 1000000;
 // The same for the count of several streams, and for the outputs of one stream
 // and of several.
 constexpr long long kCellCountShared = 60000;
-constexpr long long kCellOutputsOne = 80000;
+constexpr long long kCellOutputsOne = 400000;
 constexpr long long kCellOutputsShared = 110000;
+
+// Largest single streams merged by a wave per cell: in 2-D, in 3-D, and in 3-D
+// with reach 3, whose cells are a third of eps and so more.
+constexpr int kWaveMerge2 = 2048;
+constexpr int kWaveMerge3 = 80000;
+constexpr int kWaveMergeFine = 32000;
 
 // Uploads descriptors and prefix tables; drops a captured graph. Called when
 // the batch is built and whenever a member stream was re-initialised.
@@ -665,10 +671,12 @@ int refresh_batch(rtdbs_batch *b) {
     // windows fill the device's lanes. us cell / point (the point count with the
     // pass over the cells that follows it): several streams count 36,000 points
     // 11.6 / 12.5, 91,000 20.6 / 16.9, 338,000 59 / 38; outputs 91,000 20.4 / 23.7,
-    // 125,000 26.2 / 24.5, 338,000 58 / 33. One stream's outputs: 61,500 3-D
-    // points 9.7 / 12.5, 100,000 12.6 / 11.1 and 10.7 / 4.7 in 1-D, 14.0 / 13.1 in
-    // 2-D, 500,000 54 / 29; its count only above kCellParMaxPoints (200,000 3-D
-    // points 23.5 / 29.2, 500,000 48 / 56, one million uneven ones 123 / 116).
+    // 125,000 26.2 / 24.5, 338,000 58 / 33. One stream's outputs depend on how long
+    // its border points' stencils are, which the point form walks four lanes each:
+    // 300,000 3-D points at 1.0 eps 36 / 61, 100,000 at 0.5 12.6 / 11.1, 500,000 60 /
+    // 86 and 54 / 29, 250,000 2-D points 18 / 45, 500,000 25 / 21, 500,000 and
+    // 1 M uneven ones 82 / 61 and 116 / 73. Its count only above kCellParMaxPoints
+    // (200,000 3-D points 23.5 / 29.2, 500,000 48 / 56, 1 M uneven ones 123 / 116).
     // RTDBS_NEIGHBOR_MODE: 1 forces cell-parallel, 2 point-parallel (over a
     // single stream's own neighbor_mode).
     const int nmode = env_int("RTDBS_NEIGHBOR_MODE", 0, 0, 2);
@@ -689,10 +697,6 @@ int refresh_batch(rtdbs_batch *b) {
     b->shape.cellpar_blocks = (int)std::max(
         1ll, std::min((long long)device_cus() * env_int("RTDBS_CELLPAR_PER_CU", cp_def, 1, kMaxPerCu),
                       (cells_total + 3) / 4));
-    // merge: streams with safe cells by links and joins of cells, streams of
-    // reach 1, which have none, core by core
-    b->shape.link = b->shape.unsafe = 0;
-    for (int i = 0; i < n; i++) (b->streams[i]->dense_ok ? b->shape.link : b->shape.unsafe) = 1;
     // Cells per wave of the merge: small tiles keep a latency-bound launch's
     // waves short, large ones fill the lanes where waves abound. us of the merge
     // with 8 / 16 / 32 / 64 cells: 100,000 3-D points 27 / 28 / 35 / 38; 110,000
@@ -701,7 +705,20 @@ int refresh_batch(rtdbs_batch *b) {
     // 114; 3.2 M of 64 streams - / 234 / 168 / 138. RTDBS_CELL_TILE overrides.
     const int ctile_def =
         cells_total <= 100000 ? 8 : (cells_total <= 250000 ? 16 : (cells_total <= 2000000 ? 32 : 64));
-    const int ctile = env_int("RTDBS_CELL_TILE", ctile_def, 1, 64);
+    const int ctile_env = env_int("RTDBS_CELL_TILE", 0, 1, 64);
+    const int ctile = ctile_env ? ctile_env : ctile_def;
+    // Merge: by links and joins of tiles of cells, or by a wave per cell, whose
+    // chain is shorter, for streams of reach 1 and for a single stream of few
+    // points (both sides' times at union_cell; from 2,000 2-D points on the
+    // links and joins win). RTDBS_WAVE_MERGE forces either for streams of more
+    // reach, RTDBS_CELL_TILE the links and joins.
+    const rtdbs_params &q0 = b->streams[0]->p;
+    const int wave = env_int("RTDBS_WAVE_MERGE", -1, 0, 1);
+    const int wave_most =
+        q0.dim == 3 ? (b->streams[0]->k >= 3 ? kWaveMergeFine : kWaveMerge3) : (q0.dim == 2 ? kWaveMerge2 : 0);
+    const bool wave_merge = wave >= 0 ? wave : !ctile_env && n == 1 && q0.window <= wave_most;
+    b->shape.link = b->shape.by_wave = 0;
+    for (int i = 0; i < n; i++) (b->streams[i]->dense_ok && !wave_merge ? b->shape.link : b->shape.by_wave) = 1;
     b->shape.link_blocks =
         (int)std::max(1ll, std::min((long long)device_cus() * 16, (cells_total + 4 * ctile - 1) / (4 * ctile)));
     // lanes per query: enough threads to cover the device several times over,
@@ -734,6 +751,7 @@ int refresh_batch(rtdbs_batch *b) {
     a.cell_pre = b->d_cell_pre;
     a.ctile_pre = b->d_ctile_pre;
     a.cell_tile = ctile;
+    a.wave_merge = wave_merge;
     // XCD-grouped work order: in large batches for the merge and the
     // point-parallel output kernel, where it pays (RTDBS_XCD_GROUPS sets the
     // kXcd* bits)

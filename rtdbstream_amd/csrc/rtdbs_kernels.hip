@@ -1671,8 +1671,8 @@ __device__ __forceinline__ CellHdr load_hdr(const StreamDev &S, int A) {
 // million points, 86 to 76 at 24 served streams. (A tile of 512 positions
 // regrouped together instead of 64: 138, 89 and 91 us. Eight and 16 lanes a
 // point instead of four: 144 and 178, 91 and 100, 101 and 128.)
-__device__ __forceinline__ uint8_t count_flags(int cnt, int minpts) {
-    return cnt >= minpts ? kFlagCore : (cnt <= 1 ? kFlagAlone : 0);
+__device__ __forceinline__ uint8_t count_flags(int cnt, int minpts, bool safe) {
+    return cnt >= minpts ? (safe ? kFlagCore : kFlagCore | kFlagLoose) : (cnt <= 1 ? kFlagAlone : 0);
 }
 
 // A point that needs no look at its stencil to be noise. (The work counters
@@ -1774,7 +1774,7 @@ __device__ __forceinline__ void count_cell(const CellView &V, int A, const CellH
             test(jb, x, y, z);
         }
         if (lane < nq) {
-            V.flags[cs + q0 + lane] = count_flags(mine, minpts);
+            V.flags[cs + q0 + lane] = count_flags(mine, minpts, safe);
             // unsafe cell: every core its own element
             if (!safe) V.uf[V.W + cs + q0 + lane] = ufe(qslot, V.W + cs + q0 + lane);
         }
@@ -1963,15 +1963,18 @@ constexpr int kEdgeCap = 320;
 // One cell's header as the merge needs it: stream, cell within the stream,
 // first core position (kNoCore: none, or no cell) and position range.
 struct CellHead {
-    int s, c, fc, cs, ce;
+    int s, c, fc, cf, cs, ce;
 };
+
+// Streams whose cells the one-wave-per-cell merge unites.
+__device__ __forceinline__ bool merged_by_wave(const BatchArgs &a, int dense_ok) { return a.wave_merge || !dense_ok; }
 
 // Lane l's cell g = g0 + l * nw of a wave's grid-stride sequence: its stream
 // by a per-lane binary search over the batch's cell prefix (a small table
 // that stays in cache), then the header, all lanes' loads in one round. A cell
 // past `total`, or of a stream with safe cells, reads as a cell without cores.
 __device__ __forceinline__ CellHead cell_head(const BatchArgs &a, long long g, int total) {
-    CellHead h{0, 0, kNoCore, 0, 0};
+    CellHead h{0, 0, kNoCore, 0, 0, 0};
     bool valid = g < total;
     const gptr<const int32_t> pre = gl((const int32_t *)a.cell_pre);
     int lo = 0, hi = a.n, plo = 0;  // pre[0] = 0
@@ -1988,8 +1991,9 @@ __device__ __forceinline__ CellHead cell_head(const BatchArgs &a, long long g, i
     h.s = lo;
     h.c = valid ? (int)(g - plo) : 0;
     const gptr<const StreamDev> sd = gl(a.s) + h.s;
-    valid = valid && !sd->dense_ok;
+    valid = valid && merged_by_wave(a, sd->dense_ok);
     if (valid) {
+        h.cf = gl((const uint8_t *)sd->cflag)[h.c];
         h.fc = gl((const int32_t *)sd->fcore)[h.c];
         h.cs = gl((const int32_t *)sd->cstart)[h.c];
         h.ce = gl((const int32_t *)sd->cstart)[h.c + 1];
@@ -1999,7 +2003,7 @@ __device__ __forceinline__ CellHead cell_head(const BatchArgs &a, long long g, i
 
 // Lane j's header, wave-uniform.
 __device__ __forceinline__ CellHead lane_head(const CellHead &m, int j) {
-    return CellHead{lane_i(m.s, j), lane_i(m.c, j), lane_i(m.fc, j), lane_i(m.cs, j), lane_i(m.ce, j)};
+    return CellHead{lane_i(m.s, j), lane_i(m.c, j), lane_i(m.fc, j), lane_i(m.cf, j), lane_i(m.cs, j), lane_i(m.ce, j)};
 }
 
 struct Edge {
@@ -2020,31 +2024,70 @@ __device__ __forceinline__ void edge_flush(const BatchArgs &a, EdgeBuf &eb) {
     eb.n = 0;
 }
 
+// Queues (target, rep) for every lane that wants it, once per run of lanes
+// holding the same element (a safe cell's points are adjacent in a candidate
+// chunk and share one).
 template <class ST>
-__device__ __forceinline__ void edge_push(const BatchArgs &a, EdgeBuf &eb, int s, bool want, int x, int y, ST &st) {
+__device__ __forceinline__ void unite_once_per_rep(const BatchArgs &a, EdgeBuf &eb, int s, bool want, int rep,
+                                                   int target, ST &st) {
+    const int lane = lane_id();
     const uint64_t m = __ballot(want);
     if (m == 0ull) return;
-    const int n = __popcll(m);
-    st.add(kStatMergePairs, n);
-    st.add(kStatUnites, n);
-    if (eb.n + n > kEdgeCap) edge_flush(a, eb);
-    if (want) eb.e[eb.n + __popcll(m & ((1ull << lane_id()) - 1ull))] = Edge{x, y, s};
-    eb.n += n;
+    const uint64_t below = m & ((1ull << lane) - 1ull);
+    const int prev = below ? 63 - __clzll((long long)below) : lane;
+    const int prep = __shfl(rep, prev);
+    const bool first = want && (below == 0ull || prep != rep);
+    const uint64_t fm = __ballot(first);
+    const int nf = __popcll(fm);
+    st.add(kStatMergePairs, __popcll(m));
+    st.add(kStatUnites, nf);
+    if (eb.n + nf > kEdgeCap) edge_flush(a, eb);
+    if (first) eb.e[eb.n + __popcll(fm & ((1ull << lane) - 1ull))] = Edge{target, rep, s};
+    eb.n += nf;
 }
 
-// The cores of cell A against the stencil's cores before them in the window
-// (the reference's __raygen__cluster + unite, dbscan.cu:279-321,354-394,9-43),
-// one wave per cell: the candidates 64 at a time, coalesced, each core tested
-// against all of them with one ballot. The stencil rows (rw, lane r: row r)
-// came in with the previous cell.
+// Candidate positions before which a safe cell's merge goes over candidate
+// cells first (below it, scanning the positions costs fewer round trips).
+constexpr int kCellLevelMin = 192;
+
+// Cluster merge (the reference's __raygen__cluster + unite,
+// dbscan.cu:279-321,354-394,9-43) by one wave per cell A with cores, for
+// streams of reach 1, which have no safe cell, and for a single small stream.
+// A's candidates are the stencil positions before A's own first position - the
+// points of the stencil cells ordered before A, so each pair of cells is
+// tested once, from its later cell - loaded 64 at a time, coalesced. A safe
+// cell is one element: a candidate core within eps of any core of A joins it.
+// The cores of an unsafe cell are separate elements (kFlagLoose), and the
+// cell's own earlier points are candidates too.
+//
+// It is bound by its chain of loads, which is shorter than that of the links
+// and joins (k_merge_cells), but it tests the cores of every pair. us of both:
+// 3-D trajectories of 3,474 points 9.2 and 17.8, 20,588 points 11.5 and 20.8,
+// 30,740 14.2 and 17.2, 33,750 21.6 and 18.5, 34,240 at a third of eps 32.6 and
+// 21.1, 40,440 16.5 and 24.2, 49,221 19.5 and 19.6, 76,272 23.6 and 28.2; 2-D blobs of 831 points 8.1
+// and 13.0, 10,000 28.6 and 14.7; 100,000 1-D points 128 and 15. Six waves a
+// SIMD, not eight: no spills, and few waves in such a launch (3,474 points 10.4
+// us with eight, 34,240 35.8).
+//
+// A safe cell with many candidates goes over its candidate cells first, 64 per
+// round: a safe candidate cell joins A as soon as its first core is within eps
+// of a core of A. Only the cells not settled that way have their points
+// scanned.
 template <class ST>
 __device__ void union_cell(const BatchArgs &a, int s, const CellView &V, const CellHead &h, ST &st, EdgeBuf &eb,
                            uint64_t rw) {
     const int lane = lane_id();
     const int dim = V.dim;
     const float e2 = V.eps2;
+    // the header comes screened (cell_head) and the stencil rows (rw, lane r:
+    // row r, every lane loaded) came in with the previous cell; the first
+    // queries and the first candidate chunk load in one round, then each
+    // further chunk is a round of its own
+    const bool safeA = h.cf & kCellSafe;
     const int cs = h.cs, nA = h.ce - h.cs;
-    const RowWalk w0 = row_walk(lane < V.R ? rw : 0ull, cs + nA);
+    const RowWalk w0 = row_walk(lane < V.R ? rw : 0ull, safeA ? cs : cs + nA);
+    if (w0.rest == 0ull) return;
+    const bool by_cells = safeA && uni(wave_sum(w0.len)) >= kCellLevelMin;
     for (int q0 = 0; q0 < nA; q0 += 64) {
         const int nq = min(64, nA - q0);
         const int pq = cs + q0 + min(lane, nq - 1);
@@ -2052,34 +2095,157 @@ __device__ void union_cell(const BatchArgs &a, int s, const CellView &V, const C
         const float qx = V.sx[pq];
         const float qy = dim > 1 ? V.sy[pq] : 0.f;
         const float qz = dim > 2 ? V.sz[pq] : 0.f;
-        const uint64_t qm = __ballot(lane < nq && (qf & kFlagCore));
+        // the point scan's first chunk, in the same round (not for the
+        // cell-level pass, which scans other walks)
+        RowWalk w1 = w0;
+        int end1 = 0;
+        const int pos1 = walk_chunk(w1, 0, &end1);
+        const int f1 = by_cells ? 0 : V.flags[pos1];
+        const float x1 = by_cells ? 0.f : V.sx[pos1];
+        const float y1 = by_cells || dim < 2 ? 0.f : V.sy[pos1];
+        const float z1 = by_cells || dim < 3 ? 0.f : V.sz[pos1];
+        const int r1 = by_cells ? 0 : V.pcell[pos1];
+        arrived(qx);
+        arrived(qy);
+        arrived(qz);
+        arrived(x1);
+        arrived(y1);
+        arrived(z1);
+        arrived(r1);
+        const bool qcore = lane < nq && (qf & kFlagCore);
+        const uint64_t qm = __ballot(qcore);
         if (qm == 0ull) continue;
-        RowWalk w = w0;
-        for (int jb = 0;; jb += 64) {
-            int end;
-            const int pos = walk_chunk(w, jb, &end);
-            if (jb >= end) break;
-            const int f = V.flags[pos];
-            const float cx = V.sx[pos];
-            const float cy = dim > 1 ? V.sy[pos] : 0.f;
-            const float cz = dim > 2 ? V.sz[pos] : 0.f;
-            arrived(cx);
-            arrived(cy);
-            arrived(cz);
-            const bool bcore = jb + lane < end && (f & kFlagCore);
-            for (uint64_t m = qm; m; m &= m - 1ull) {
-                const int qi = __ffsll((unsigned long long)m) - 1;
-                st.add(kStatMergeTests, (unsigned)min(64, end - jb));
-                const bool hit = bcore & (pos < cs + q0 + qi) &
-                                 (sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2);
-                edge_push(a, eb, s, hit, V.W + pos, V.W + cs + q0 + qi, st);
+        // The cores qm of this block against candidate chunk [jb, jb + 64) of
+        // a walk whose candidates end at `end`.
+        auto test = [&](const int jb, const int end, const int pos, const int f, const float cx, const float cy,
+                        const float cz, const int rp) __attribute__((always_inline)) {
+                const bool bcore = jb + lane < end && (f & kFlagCore);
+                const uint64_t bm = __ballot(bcore);
+                if (bm == 0ull) return;
+                const int rep = bcore ? ((f & kFlagLoose) ? V.W + pos : rp) : -1;
+                const unsigned chunk = (unsigned)min(64, end - jb);
+                uint64_t m = qm;
+                if (safeA) {
+                    // lanes holding one element form a run (a safe cell's points are
+                    // adjacent); one touching lane settles its whole run
+                    const int prev_rep = prev_lane(rep);  // every lane takes part in the moves
+                    const int prev_core = prev_lane((int)bcore);
+                    const uint64_t starts = __ballot(lane == 0 || prev_rep != rep || !prev_core);
+                    const uint64_t after = starts & ~((2ull << lane) - 1ull);  // run starts above this lane
+                    const uint64_t upto = after ? (after & (~after + 1ull)) - 1ull : ~0ull;
+                    const uint64_t below = starts & ((2ull << lane) - 1ull);
+                    const uint64_t from = ~((1ull << (63 - __clzll((long long)below))) - 1ull);
+                    const uint64_t run = upto & from;  // this lane's run
+                    // touched candidates as one wave mask: the loop carries a scalar,
+                    // not a lane predicate
+                    uint64_t t = 0;
+                    while (m) {
+                        const int qi = __ffsll((unsigned long long)m) - 1;
+                        m &= m - 1;
+                        st.add(kStatMergeTests, chunk);
+                        // every lane evaluates the test, no branch per query
+                        t |= __ballot(sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2) & bm;
+                        if ((__ballot((t & run) != 0ull) | ~bm) == ~0ull) break;  // every candidate run settled
+                    }
+                    unite_once_per_rep(a, eb, s, (t >> lane) & 1ull, rep, h.c, st);
+                } else {
+                    while (m) {
+                        const int qi = __ffsll((unsigned long long)m) - 1;
+                        m &= m - 1;
+                        st.add(kStatMergeTests, chunk);
+                        const bool hit = bcore & (pos < cs + q0 + qi) &
+                                         (sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), cx, cy, cz) < e2);
+                        unite_once_per_rep(a, eb, s, hit, rep, V.W + cs + q0 + qi, st);
+                    }
+                }
+        };
+        // the cores qm of this block against the candidate positions of walk w
+        auto scan = [&](RowWalk w) __attribute__((always_inline)) {
+            for (int jb = 0;; jb += 64) {
+                int end;
+                const int pos = walk_chunk(w, jb, &end);
+                if (jb >= end) break;
+                const int f = V.flags[pos];
+                const float cx = V.sx[pos];
+                const float cy = dim > 1 ? V.sy[pos] : 0.f;
+                const float cz = dim > 2 ? V.sz[pos] : 0.f;
+                const int rp = V.pcell[pos];
+                arrived(cx);
+                arrived(cy);
+                arrived(cz);
+                arrived(rp);
+                test(jb, end, pos, f, cx, cy, cz, rp);
             }
+        };
+        if (!by_cells) {
+            // the first chunk came with the queries
+            if (end1 > 0) test(0, end1, pos1, f1, x1, y1, z1, r1);
+            for (int jb = 64;; jb += 64) {
+                int end;
+                const int pos = walk_chunk(w1, jb, &end);
+                if (jb >= end) break;
+                const int f = V.flags[pos];
+                const float cx = V.sx[pos];
+                const float cy = dim > 1 ? V.sy[pos] : 0.f;
+                const float cz = dim > 2 ? V.sz[pos] : 0.f;
+                const int rp = V.pcell[pos];
+                arrived(cx);
+                arrived(cy);
+                arrived(cz);
+                arrived(rp);
+                test(jb, end, pos, f, cx, cy, cz, rp);
+            }
+            continue;
+        }
+        // candidate cells: row r (lane r) covers positions [rx, rx + len), all
+        // before cs, i.e. the cells pcell[rx] .. pcell[rx + len - 1] (< A)
+        const int clo = w0.len > 0 ? V.pcell[w0.rx] : 0;
+        const int chi = w0.len > 0 ? V.pcell[w0.rx + w0.len - 1] + 1 : 0;
+        RowWalk cw;
+        cw.rx = clo;
+        cw.len = chi - clo;
+        cw.rest = __ballot(cw.len > 0);
+        for (int jb = 0;; jb += 64) {
+            int endc;
+            const int B = walk_chunk(cw, jb, &endc);
+            if (jb >= endc) break;
+            const bool valid = jb + lane < endc;
+            const int fb = V.fcore[B];
+            const int cfb = V.cflag[B];
+            const int bs = V.cstart[B];
+            const int be = V.cstart[B + 1];
+            arrived(fb);
+            arrived(be);
+            const bool has = valid && fb != kNoCore;
+            const int fp = has ? fb : cs;  // a valid position either way
+            const float bx = V.sx[fp];
+            const float by = dim > 1 ? V.sy[fp] : 0.f;
+            const float bz = dim > 2 ? V.sz[fp] : 0.f;
+            arrived(bx);
+            arrived(by);
+            arrived(bz);
+            // safe candidate cells: A's cores against each cell's first core
+            const uint64_t cand = __ballot(has && (cfb & kCellSafe));
+            uint64_t hit = 0;
+            for (uint64_t m = qm; m && hit != cand;) {
+                const int qi = __ffsll((unsigned long long)m) - 1;
+                m &= m - 1;
+                st.add(kStatMergeTests, (unsigned)__popcll(cand & ~hit));
+                hit |= __ballot(sqd(dim, lane_f(qx, qi), lane_f(qy, qi), lane_f(qz, qi), bx, by, bz) < e2) & cand;
+            }
+            unite_once_per_rep(a, eb, s, (hit >> lane) & 1ull, B, h.c, st);
+            // the cells with cores not settled: scan their points
+            RowWalk pw;
+            pw.rx = bs;
+            pw.len = (has && !((hit >> lane) & 1ull)) ? be - bs : 0;
+            pw.rest = __ballot(pw.len > 0);
+            if (pw.rest) scan(pw);
         }
     }
 }
 
 template <class ST>
-__global__ __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_union(BatchArgs a) {
+__global__ __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_union(BatchArgs a) {
     __shared__ Edge edges[kCellWaves][kEdgeCap];
     const int total = uni(ldc(a.cell_pre[a.n]));
     const int nw = gridDim.x * kCellWaves;
@@ -2653,7 +2819,7 @@ __device__ __forceinline__ void each_cell_tile(const BatchArgs &a, ST &st, F &&t
          g < total; g += nw) {
         s = uni(find_stream_from(a.ctile_pre, a.n, g, s));
         const StreamDev &S = a.s[s];
-        if (!ldc(S.dense_ok)) continue;
+        if (merged_by_wave(a, ldc(S.dense_ok))) continue;
         stats_stream(a, st, s);
         tile(S, cell_view(S), (g - uni(ldc(a.ctile_pre[s]))) * a.cell_tile, ldc(ldc(S.mut)->ncell));
     }
@@ -2826,7 +2992,7 @@ __device__ __forceinline__ void count_vblock(const BatchArgs &a, const QueryLane
     }
     cnt = group_sum<LPQ>(cnt);
     if (valid && ql.sub == 0) {
-        V.flags[p] = dense ? (kFlagCore | kFlagDense) : count_flags(cnt, minpts);
+        V.flags[p] = dense ? (kFlagCore | kFlagDense) : count_flags(cnt, minpts, safe);
         if (!safe) V.uf[V.W + p] = ufe(vslot(V, p), V.W + p);  // a core of an unsafe cell is an element
     }
 }
@@ -3222,8 +3388,8 @@ hipError_t launch_slide(const BatchArgs &a, const LaunchShape &sh, hipStream_t s
     if (!sh.count_cell) RTDBS_LAUNCH(k_cell_cores, sh.link_blocks, 64 * kCellWaves, a);
     if (sh.link && a.stats) RTDBS_LAUNCH(k_merge_cells<WaveStats>, sh.link_blocks, 64 * kCellWaves, a);
     else if (sh.link) RTDBS_LAUNCH(k_merge_cells<NoStats>, sh.link_blocks, 64 * kCellWaves, a);
-    if (sh.unsafe && a.stats) RTDBS_LAUNCH(k_union<WaveStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
-    else if (sh.unsafe) RTDBS_LAUNCH(k_union<NoStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
+    if (sh.by_wave && a.stats) RTDBS_LAUNCH(k_union<WaveStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
+    else if (sh.by_wave) RTDBS_LAUNCH(k_union<NoStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
     PH_END(kPhUnion);
     PH_BEGIN(kPhBorder);
     if (sh.cellpar && a.stats) RTDBS_LAUNCH(k_border<WaveStats>, sh.cellpar_blocks, 64 * kCellWaves, a);
