@@ -251,13 +251,16 @@ __device__ __forceinline__ uint64_t ufe_root(P u, uint64_t e) {
 
 // Unites elements x and y: both walks step together, the larger root hooks
 // under the smaller by an atomic minimum (as uf_unite), and both starting
-// entries are pointed at the root afterwards.
-template <class P>
+// entries are pointed at the root afterwards. With CACHED the walks use plain
+// loads: a stale entry is an ancestor all the same, and a root that is none any
+// more shows in what the hook's atomic returns, which strictly falls.
+template <bool CACHED = false, class P>
 __device__ __forceinline__ void ufe_unite(P u, int x, int y) {
-    const uint64_t x0 = ufe_now(u, x), y0 = ufe_now(u, y);
+    auto entry = [&](int i) { return CACHED ? at(u, i) : ufe_now(u, i); };
+    const uint64_t x0 = entry(x), y0 = entry(y);
     uint64_t a = x0, b = y0;
     while (a != b) {
-        const uint64_t na = ufe_now(u, ufe_idx(a)), nb = ufe_now(u, ufe_idx(b));
+        const uint64_t na = entry(ufe_idx(a)), nb = entry(ufe_idx(b));
         if (na != a || nb != b) {
             a = na;
             b = nb;

@@ -606,11 +606,9 @@ constexpr long long kCellCountShared = 60000;
 constexpr long long kCellOutputsOne = 400000;
 constexpr long long kCellOutputsShared = 110000;
 
-// Largest single streams merged by a wave per cell: in 2-D, in 3-D, and in 3-D
-// with reach 3, whose cells are a third of eps and so more.
+// Largest single streams merged by a wave per cell, in 2-D and 3-D.
 constexpr int kWaveMerge2 = 2048;
-constexpr int kWaveMerge3 = 80000;
-constexpr int kWaveMergeFine = 32000;
+constexpr int kWaveMerge3 = 90000;
 
 // Uploads descriptors and prefix tables; drops a captured graph. Called when
 // the batch is built and whenever a member stream was re-initialised.
@@ -714,8 +712,7 @@ int refresh_batch(rtdbs_batch *b) {
     // reach, RTDBS_CELL_TILE the links and joins.
     const rtdbs_params &q0 = b->streams[0]->p;
     const int wave = env_int("RTDBS_WAVE_MERGE", -1, 0, 1);
-    const int wave_most =
-        q0.dim == 3 ? (b->streams[0]->k >= 3 ? kWaveMergeFine : kWaveMerge3) : (q0.dim == 2 ? kWaveMerge2 : 0);
+    const int wave_most = q0.dim == 3 ? kWaveMerge3 : (q0.dim == 2 ? kWaveMerge2 : 0);
     const bool wave_merge = wave >= 0 ? wave : !ctile_env && n == 1 && q0.window <= wave_most;
     b->shape.link = b->shape.by_wave = 0;
     for (int i = 0; i < n; i++) (b->streams[i]->dense_ok && !wave_merge ? b->shape.link : b->shape.by_wave) = 1;

@@ -2019,7 +2019,7 @@ struct EdgeBuf {
 __device__ __forceinline__ void edge_flush(const BatchArgs &a, EdgeBuf &eb) {
     for (int i = lane_id(); i < eb.n; i += 64) {
         const Edge e = eb.e[i];
-        ufe_unite(gl(ldc(a.s[e.s].uf)), e.x, e.y);
+        ufe_unite<true>(gl(ldc(a.s[e.s].uf)), e.x, e.y);
     }
     eb.n = 0;
 }
@@ -2062,12 +2062,13 @@ constexpr int kCellLevelMin = 192;
 //
 // It is bound by its chain of loads, which is shorter than that of the links
 // and joins (k_merge_cells), but it tests the cores of every pair. us of both:
-// 3-D trajectories of 3,474 points 9.2 and 17.8, 20,588 points 11.5 and 20.8,
-// 30,740 14.2 and 17.2, 33,750 21.6 and 18.5, 34,240 at a third of eps 32.6 and
-// 21.1, 40,440 16.5 and 24.2, 49,221 19.5 and 19.6, 76,272 23.6 and 28.2; 2-D blobs of 831 points 8.1
-// and 13.0, 10,000 28.6 and 14.7; 100,000 1-D points 128 and 15. Six waves a
-// SIMD, not eight: no spills, and few waves in such a launch (3,474 points 10.4
-// us with eight, 34,240 35.8).
+// 3-D trajectories of 3,474 points 9.9 and 17.8, 20,588 points 10.7 and 20.8,
+// 33,750 19.3 and 18.5, 40,440 15.5 and 24.2, 76,272 22.7 and 28.2; at a third of
+// eps 34,240 28.6 and 21.1, 81,781 27.6 and 31.0; 2-D blobs of 831 points 8.1 and
+// 13.0, 10,000 28.6 and 14.7; 100,000 1-D points 128 and 15. Six waves a SIMD,
+// not eight: no spills, and few waves in such a launch (3,474 points 10.4 us with
+// eight). The unites walk by cached loads (agent-scope ones: 40,440 points 16.0
+// us, 81,781 30.2, 33,750 21.4).
 //
 // A safe cell with many candidates goes over its candidate cells first, 64 per
 // round: a safe candidate cell joins A as soon as its first core is within eps

@@ -46,8 +46,7 @@ def test_pairs_near_eps(engine, oracle, monkeypatch, wave, n, apart):
     _check(engine, oracle, np.concatenate([pts, pts]), 3, W, W // 2, 1.0, max(1, n // 2), 2, "n %d" % n)
 
 
-@pytest.mark.parametrize("dim,W,k", [(2, 2048, 2), (2, 2050, 2), (3, 80000, 2), (3, 80002, 2), (3, 32000, 3),
-                                     (3, 32002, 3)])
+@pytest.mark.parametrize("dim,W,k", [(2, 2048, 2), (2, 2050, 2), (3, 90000, 2), (3, 90002, 3)])
 def test_choice_by_size(engine, oracle, dim, W, k):
     S = W // 2
     data = _clumps(W + S, dim, W, W // 40, 0.4, 3.0 * W ** (1.0 / dim) / 2)
