@@ -128,9 +128,9 @@ struct LaunchShape {
     int32_t rows_blocks;     // 256-thread blocks for the row kernel
     int32_t lpq;             // lanes per query of the point-parallel count (1, 2 or 4)
     int32_t lpq_border;      // lanes per query of the point-parallel output kernel
-    int32_t cellpar_blocks;  // blocks of the cell-parallel count and border kernels
+    int32_t cellpar_blocks;  // blocks of the kernels with a wave per cell: count, border, k_union
     int32_t cellpar;         // 1: cell-parallel output kernel, 0: point-parallel
-    int32_t count_cell;      // 1: cell-parallel range count (writes fcore and rep), 0: point-parallel
+    int32_t count_cell;      // 1: cell-parallel range count (writes fcore and uf), 0: point-parallel
     int32_t link;            // 1: some stream is merged by k_merge_cells
     int32_t by_wave;         // 1: some stream is merged by k_union
     int32_t link_blocks;     // blocks of k_merge_cells and k_cell_cores

@@ -651,7 +651,8 @@ int refresh_batch(rtdbs_batch *b) {
     // (RTDBS_SMALL_UPDATE: 0 forces the separate kernels)
     b->shape.small_update =
         small && env_int("RTDBS_SMALL_UPDATE", 1, 0, 1) ? (most + kSmallThreads - 1) / kSmallThreads : 0;
-    // stride rank: 64-key blocks when 256-key blocks would not cover the device
+    // stride rank: a block's four waves split the runs for 64 keys where blocks of
+    // 256 keys, a wave for every 64, would not cover the device
     // (RTDBS_RANK_SPLIT: 0 forces 256-key blocks, 1 the 64-key form)
     const int rsplit = env_int("RTDBS_RANK_SPLIT", -1, 0, 1);
     b->shape.rank_split =
@@ -687,9 +688,9 @@ int refresh_batch(rtdbs_batch *b) {
     b->shape.count_cell =
         cmode ? (cmode == 1)
               : mode == 1 || (mode == 0 && cells_total <= (n == 1 ? kCellParMaxPoints : kCellCountShared));
-    // cell-parallel grid: 16 blocks per CU while the launch is small; 32 for
-    // large batches, where it carries the merge alone (64 streams: 455 ->
-    // ~400 us). RTDBS_CELLPAR_PER_CU overrides.
+    // grid of the kernels with a wave per cell: 16 blocks per CU while the
+    // launch is small, 32 for large batches, where only the merge by waves is
+    // left of them (64 streams 455 -> 400 us). RTDBS_CELLPAR_PER_CU overrides.
     const int cp_def =
         p1 && p1->cellpar_per_cu > 0 ? p1->cellpar_per_cu : (cells_total <= kCellParMaxPoints ? 16 : 32);
     b->shape.cellpar_blocks = (int)std::max(

@@ -4,7 +4,9 @@
 //   sort_expire (stride sort in runs + survivors per window tile) ->
 //   rank (stride rank merge + survivor compaction) -> merge_final -> cells ->
 //   rows -> count -> merge_cells -> border (outputs)
-// (large batches: count_points -> cell_cores -> merge_cells -> border_regroup).
+// (several streams and large ones: count_points -> cell_cores -> merge_cells ->
+// border_regroup; small windows: update_small instead of the first four; single
+// small streams and reach 1: union instead of merge_cells).
 // Each kernel covers all streams of the batch in one launch: a block finds its
 // stream from prefix tables of per-stream work units (tiles of positions,
 // 64-position chunks) or, for the cell kernels whose sizes are only known on
